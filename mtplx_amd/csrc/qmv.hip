@@ -21,6 +21,7 @@
 //    per wave load).
 //  * Activations are staged once per workgroup into LDS in the MFMA A-operand
 //    order, with optional fused producers: SwiGLU (silu(gate)*up) or RMSNorm.
+#include "qmv_inplace.hpp"
 #include "qmv_kernels.hpp"
 
 #include <stdarg.h>
@@ -38,7 +39,8 @@ void set_error(const char* fmt, ...) {
   va_end(ap);
 }
 
-// Expert-gathered matmul: work items (active expert slot, row tile, column
+// Expert-gathered matmul with the SwiGLU input (xmode 1; plain x runs
+// qmv_inplace_kernel): work items (active expert slot, row tile, column
 // tile) in slot-major order, taken grid-stride by a bounded grid. The number
 // of active experts is known only on the device; a grid over every expert
 // slot would dispatch mostly empty workgroups (e.g. 63 of 256 experts
@@ -413,6 +415,29 @@ MTP_API int mtp_gather_qmv_affine4(const void* x, const void* x2, const uint32_t
     set_error("%s: x and weights must be 16-byte aligned", who);
     return MTP_ERR_ARG;
   }
+  if (xmode == X_PLAIN) {
+    InplaceParams p = {};
+    p.x = (const uint16_t*)x;
+    p.w0 = (const uint8_t*)w0;
+    p.w1 = (const uint8_t*)w1;
+    p.s0 = (const uint16_t*)s0;
+    p.b0 = (const uint16_t*)b0;
+    p.s1 = (const uint16_t*)s1;
+    p.b1 = (const uint16_t*)b1;
+    p.y = (uint16_t*)y;
+    p.rowmap = rowmap;
+    p.expert_off = expert_off;
+    p.active = active;
+    p.w_estride = (long long)rows_per_expert * (K / 2);
+    p.s_estride = (long long)rows_per_expert * (K / group_size);
+    p.M = max_rows_per_expert;
+    p.N = N;
+    p.K = K;
+    p.ldx = K;
+    p.ldy = N;
+    inplace_launch(p, 4, group_size, max_rows_per_expert, emode == E_DUAL_SWIGLU, (hipStream_t)stream);
+    return launch_check(who);
+  }
   QmmParams p = base_params(x, w0, s0, b0, y, 32, N, K, group_size);
   p.x2 = (const uint16_t*)x2;
   p.w1 = (const uint32_t*)w1;
@@ -446,11 +471,7 @@ MTP_API int mtp_gather_qmv_affine4(const void* x, const void* x2, const uint32_t
     else                                                                                                     \
       hipLaunchKernelGGL((gather_qmm4_kernel<RR, XMV, EMV, 1>), grid, dim3(kThreads), pl.lds, st, p);       \
   } while (0)
-  if (xmode == X_PLAIN && emode == E_STORE) {
-    if (mrows <= 8) MTP_GATHER(4, X_PLAIN, E_STORE); else if (mrows <= 16) MTP_GATHER(8, X_PLAIN, E_STORE); else MTP_GATHER(16, X_PLAIN, E_STORE);
-  } else if (xmode == X_PLAIN) {
-    if (mrows <= 8) MTP_GATHER(4, X_PLAIN, E_DUAL_SWIGLU); else if (mrows <= 16) MTP_GATHER(8, X_PLAIN, E_DUAL_SWIGLU); else MTP_GATHER(16, X_PLAIN, E_DUAL_SWIGLU);
-  } else if (emode == E_STORE) {
+  if (emode == E_STORE) {
     if (mrows <= 8) MTP_GATHER(4, X_SWIGLU, E_STORE); else if (mrows <= 16) MTP_GATHER(8, X_SWIGLU, E_STORE); else MTP_GATHER(16, X_SWIGLU, E_STORE);
   } else {
     if (mrows <= 8) MTP_GATHER(4, X_SWIGLU, E_DUAL_SWIGLU); else if (mrows <= 16) MTP_GATHER(8, X_SWIGLU, E_DUAL_SWIGLU); else MTP_GATHER(16, X_SWIGLU, E_DUAL_SWIGLU);

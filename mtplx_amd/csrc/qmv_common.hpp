@@ -361,6 +361,39 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Direct-to-LDS loads issued as assembly: lane i's 16 (or 4) bytes go to lds +
+// 16 i (4 i); lds is a wave-uniform LDS byte address (lds_addr). With the
+// builtin the compiler takes every later LDS read of the kernel for one that
+// may need the data and waits for all loads in flight (vmcnt(0)) at the first
+// LDS read after it, which drains a double buffer at every step. These have
+// no output registers; the caller waits (wait_vm) before it reads the LDS,
+// and before it writes the same LDS again its reads have returned. A scalar
+// write of m0 needs one wait state before the load that uses it. (Nothing else
+// in these kernels uses m0, which the compiler reserves and warns about.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ uint32_t lds_addr(const void* a) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lptr_t)a);
+}
+__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {   // base wave-uniform
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :: "s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void dma16(const void* lane_ptr, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(lds), "v"(lane_ptr) : "memory", "m0");
+}
+__device__ __forceinline__ void dma4(const void* lane_ptr, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+               :: "s"(lds), "v"(lane_ptr) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+// Waits until at most N vector-memory operations of the wave are in flight.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+
 // s_waitcnt immediate for "at most vm vector-memory ops outstanding" (gfx9
 // encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] at 15:14).
 __host__ __device__ constexpr int vmcnt_imm(int vm) { return (vm & 0xF) | (0x7 << 4) | (0xF << 8) | ((vm >> 4) << 14); }
