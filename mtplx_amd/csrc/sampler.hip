@@ -27,8 +27,10 @@
 //     accept loop. (Vocabularies over 64 chunks use accept_finish, one wave
 //     per request building the laws in turn.)
 // Laws whose support may exceed 64 ids (top_k = 0 or > 64: pure nucleus, or
-// no truncation at all) take the wide path: one 1024-thread workgroup per row
-// finds the support's cut by a radix descent over the logits' order-preserving
+// no truncation at all) take the wide path. Vocabularies of more than two
+// chunks first bin every id by its distance from the row's maximum over many
+// workgroups (wide_hist), which leaves one bin to cut; small ones skip that.
+// One 1024-thread workgroup per row finds the support's cut by a radix descent over the logits' order-preserving
 // bits (four 8-bit passes of per-digit counts and probability mass, the mass
 // in 2^-62 fixed point so integer atomics keep it exact and order-free),
 // resolves the cut inside the final tie group by id, and writes the support in
@@ -52,7 +54,8 @@ namespace mtp {
 __global__ __launch_bounds__(kSampThreads) void vocab_partials(const float* __restrict__ logits,
                                                                const float* __restrict__ logits2, int nrows1,
                                                                long long ld, int V, int n_chunks, double temp,
-                                                               int ksel, int greedy, ChunkPart* __restrict__ parts) {
+                                                               int ksel, int greedy, ChunkPart* __restrict__ parts,
+                                                               uint32_t* __restrict__ zero, int zero_words) {
   constexpr int NWV = kSampThreads / 64;
   static_assert(NWV == 8, "the list merge reduces over 8 lanes");
   const int chunk = blockIdx.x;
@@ -62,6 +65,10 @@ __global__ __launch_bounds__(kSampThreads) void vocab_partials(const float* __re
   const int wave = tid >> 6;
   const float* lr = row < nrows1 ? logits + (size_t)row * ld : logits2 + (size_t)(row - nrows1) * ld;
   const int base = chunk * kChunk;
+  // The wide path's histograms of this row, cleared for the launch that adds to them.
+  if (zero)
+    for (int i = chunk * kSampThreads + tid; i < zero_words; i += n_chunks * kSampThreads)
+      zero[(size_t)row * zero_words + i] = 0u;
 
   float v[kEPT];
   double qv[kEPT];   // l / T in fp64, computed once
@@ -121,6 +128,30 @@ __global__ __launch_bounds__(kSampThreads) void vocab_partials(const float* __re
   for (int e = 0; e < kEPT; ++e) {
     const int id = base + e * kSampThreads + tid;
     keys[e] = (id < V && !isnan(v[e])) ? make_key(v[e], id) : 0ull;
+  }
+  if (ksel == 1) {
+    // The largest key alone (greedy rows, the wide path): 28 rows of 151936 in
+    // 15.1 us, 23.1 through the select below.
+    uint64_t best = 0ull;
+#pragma unroll
+    for (int e = 0; e < kEPT; ++e) best = umax64(best, keys[e]);
+    best = wave_max_u64(best);
+    __shared__ uint64_t s_best[NWV];
+    if (lane == 0) s_best[wave] = best;
+    __syncthreads();
+    if (tid == 0) {
+      ChunkPart* out = parts + (size_t)row * n_chunks + chunk;
+      int nf = 0;
+      for (int w = 0; w < NWV; ++w) {
+        best = umax64(best, s_best[w]);
+        nf |= s_nf[w];
+      }
+      out->keys[0] = best;
+      out->m = mchunk;
+      out->s = schunk;
+      out->nonfinite = nf;
+    }
+    return;
   }
   __shared__ int s_hist[256];
   __shared__ uint64_t s_sel[kMaxTopK];
@@ -1228,6 +1259,468 @@ __global__ __launch_bounds__(kWideThreads) void wide_law_kernel(const float* __r
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same law over many workgroups, for rows of more than two chunks. One
+// workgroup per row leaves most of the chip idle (28 rows on 256 CUs) and walks
+// a row in 149 rounds of block scans: 557 us for 28 rows of 151936. Here, with
+// the same ids and probabilities bit for bit, 24 + 15 + 14 + 34 us (four
+// requests' accept step of depth 3: 597 -> 124 us):
+//  1. wide_hist: per chunk, the count and fixed-point mass of each bin of the
+//     distance from the row's maximum (bins are monotone in the logit; integer
+//     sums, so the order of the additions does not matter);
+//  2. wide_count, wide_collect: per chunk, the ids in the bins down to the one
+//     that holds the cut, counted, then written in id order with their
+//     probabilities (the cut bin's marked by the sign);
+//  3. wide_finish: per row, the radix descent among the cut bin's ids alone,
+//     then the support compacted in place, summed and normalised.
+constexpr int kWideBins = 1024;
+constexpr double kWideBinScale = 32.0;   // bins of 1/32 in l/T; the last one takes the rest
+// Per row: header, bin masses, bin counts, chunk counts (32-bit words from the start).
+struct WideCut {
+  double M, S;
+  unsigned long long m_above;   // mass and count above the cut bin
+  uint32_t c_above;
+  int nonfinite;
+  int bin;                      // the cut bin; kWideBins: everything is inside the cut
+  int argmax;
+  int pad[4];
+};
+constexpr int kWideCutWords = 16;
+static_assert(sizeof(WideCut) <= 4 * kWideCutWords, "the header's words");
+constexpr int kWideHistWords = kWideCutWords + 3 * kWideBins;   // the part cleared on every call
+__host__ __device__ inline size_t wide_hist_row_words(int n_chunks) {
+  return (size_t)((kWideHistWords + n_chunks + 63) & ~63);
+}
+struct WideRow {
+  WideCut* cut;
+  unsigned long long* mass;
+  uint32_t* cnt;
+  uint32_t* chunk_n;
+};
+__device__ __forceinline__ WideRow wide_row(uint32_t* hist, int n_chunks, int row) {
+  uint32_t* r = hist + wide_hist_row_words(n_chunks) * row;
+  WideRow o;
+  o.cut = reinterpret_cast<WideCut*>(r);
+  o.mass = reinterpret_cast<unsigned long long*>(r + kWideCutWords);
+  o.cnt = r + kWideCutWords + 2 * kWideBins;
+  o.chunk_n = r + kWideHistWords;
+  return o;
+}
+__device__ __forceinline__ int wide_bin(float l, double temp, double M) {
+  return (int)fmin((M - (double)l / temp) * kWideBinScale, (double)(kWideBins - 1));
+}
+__device__ __forceinline__ const float* wide_logits(const float* logits, const float* logits2, int nrows1,
+                                                    long long ld, int row) {
+  return row < nrows1 ? logits + (size_t)row * ld : logits2 + (size_t)(row - nrows1) * ld;
+}
+
+__global__ __launch_bounds__(kSampThreads) void wide_hist(const float* __restrict__ logits,
+                                                          const float* __restrict__ logits2, int nrows1, long long ld,
+                                                          int V, const ChunkPart* __restrict__ parts, int n_chunks,
+                                                          double temp, uint32_t* __restrict__ hist) {
+  constexpr int NWV = kSampThreads / 64;
+  const int chunk = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+  const float* lr = wide_logits(logits, logits2, nrows1, ld, row);
+  const ChunkPart* pp = parts + (size_t)row * n_chunks;
+  const WideRow wr = wide_row(hist, n_chunks, row);
+  __shared__ unsigned long long s_mass[kWideBins];
+  __shared__ uint32_t s_cnt[kWideBins];
+  __shared__ double s_wm[NWV], s_term[kSampThreads];
+  __shared__ int s_wnf[NWV];
+  __shared__ uint64_t s_wk[NWV];
+  __shared__ double s_S;
+  __shared__ int s_nf;
+  for (int i = tid; i < kWideBins; i += kSampThreads) {
+    s_mass[i] = 0ull;
+    s_cnt[i] = 0u;
+  }
+  float v[kEPT];
+#pragma unroll
+  for (int e = 0; e < kEPT; ++e) {
+    const int id = chunk * kChunk + e * kSampThreads + tid;
+    v[e] = id < V ? lr[id] : 0.f;
+  }
+  // fp64 max / sum-exp combine in fixed chunk order (as build_law).
+  double M = -INFINITY;
+  int nf = 0;
+  uint64_t best = 0ull;
+  for (int c = tid; c < n_chunks; c += kSampThreads) {
+    M = fmax(M, pp[c].m);
+    nf |= pp[c].nonfinite;
+    best = umax64(best, pp[c].keys[0]);
+  }
+  M = wave_max_f64(M);
+  nf = __any(nf) ? 1 : 0;
+  best = wave_max_u64(best);
+  if ((tid & 63) == 0) {
+    s_wm[tid >> 6] = M;
+    s_wnf[tid >> 6] = nf;
+    s_wk[tid >> 6] = best;
+  }
+  __syncthreads();
+  nf = 0;
+  for (int w = 0; w < NWV; ++w) {
+    M = fmax(M, s_wm[w]);
+    nf |= s_wnf[w];
+    best = umax64(best, s_wk[w]);
+  }
+  double S = 0.0;
+  for (int c0 = 0; c0 < n_chunks; c0 += kSampThreads) {
+    const int c = c0 + tid;
+    s_term[tid] = (c < n_chunks && pp[c].m > -INFINITY) ? pp[c].s * exp(pp[c].m - M) : 0.0;
+    __syncthreads();
+    if (tid == 0) {
+      const int n = n_chunks - c0 < kSampThreads ? n_chunks - c0 : kSampThreads;
+      for (int i = 0; i < n; ++i) S += s_term[i];
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    s_S = S;
+    s_nf = nf || !(isfinite(S) && S > 0.0);
+    if (chunk == 0) {
+      wr.cut->M = M;
+      wr.cut->S = S;
+      wr.cut->nonfinite = s_nf;
+      wr.cut->argmax = key_id(best);
+    }
+  }
+  __syncthreads();
+  if (s_nf) return;
+  S = s_S;
+#pragma unroll
+  for (int e = 0; e < kEPT; ++e) {
+    const int id = chunk * kChunk + e * kSampThreads + tid;
+    if (id < V) {
+      const int b = wide_bin(v[e], temp, M);
+      const double pv = exp((double)v[e] / temp - M) / S;
+      atomicAdd(&s_cnt[b], 1u);
+      const unsigned long long P = (unsigned long long)(pv * kFix62);
+      if (P) atomicAdd(&s_mass[b], P);
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < kWideBins; i += kSampThreads)
+    if (s_cnt[i]) {
+      atomicAdd(wr.cnt + i, s_cnt[i]);
+      if (s_mass[i]) atomicAdd(wr.mass + i, s_mass[i]);
+    }
+}
+
+// Chunk's ids in bins <= the row's cut bin, in id order: counted (COLLECT
+// false) or written after those of the chunks before it. The cut bin is the
+// first, from the top, after which an id is excluded (top-k full or nucleus
+// mass reached); every workgroup finds it from the row's histogram.
+template <bool COLLECT>
+__global__ __launch_bounds__(kSampThreads) void wide_collect(const float* __restrict__ logits,
+                                                             const float* __restrict__ logits2, int nrows1,
+                                                             long long ld, int V, int n_chunks, double temp, int k_eff,
+                                                             double top_p, uint32_t* __restrict__ hist,
+                                                             unsigned char* __restrict__ lawbuf, size_t row_bytes) {
+  constexpr int NWV = kSampThreads / 64;
+  constexpr int BPT = kWideBins / kSampThreads;   // bins per thread
+  const int chunk = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const float* lr = wide_logits(logits, logits2, nrows1, ld, row);
+  const WideRow wr = wide_row(hist, n_chunks, row);
+  if (wr.cut->nonfinite) return;
+  const double M = wr.cut->M, S = wr.cut->S;
+  float v[kEPT];
+#pragma unroll
+  for (int e = 0; e < kEPT; ++e) {
+    const int id = chunk * kChunk + e * kSampThreads + tid;
+    v[e] = id < V ? lr[id] : 0.f;
+  }
+  __shared__ int s_bin, s_base;
+  __shared__ uint32_t s_n[kEPT][NWV];
+  if constexpr (!COLLECT) {
+    __shared__ unsigned long long s_m[NWV];
+    __shared__ uint32_t s_c[NWV];
+    const bool nuc = top_p > 0.0 && top_p < 1.0;
+    const unsigned long long TP = nuc ? (unsigned long long)(top_p * kFix62) : ~0ull;
+    if (tid == 0) s_bin = kWideBins;
+    uint32_t c[BPT], ct = 0;
+    unsigned long long m[BPT], mt = 0ull;
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+      c[j] = wr.cnt[BPT * tid + j];
+      m[j] = wr.mass[BPT * tid + j];
+      ct += c[j];
+      mt += m[j];
+    }
+    uint32_t ci = ct;
+    unsigned long long mi = mt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(ci, o, 64);
+      const unsigned long long z = __shfl_up(mi, o, 64);
+      if (lane >= o) {
+        ci += y;
+        mi += z;
+      }
+    }
+    if (lane == 63) {
+      s_c[wave] = ci;
+      s_m[wave] = mi;
+    }
+    __syncthreads();
+    uint32_t ca = ci - ct;   // above this thread's first bin
+    unsigned long long ma = mi - mt;
+    for (int w = 0; w < wave; ++w) {
+      ca += s_c[w];
+      ma += s_m[w];
+    }
+    int hit = kWideBins;
+    uint32_t hc = 0;
+    unsigned long long hm = 0ull;
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+      if (hit == kWideBins && c[j] && ((int)(ca + c[j]) >= k_eff || (nuc && ma + m[j] >= TP))) {
+        hit = BPT * tid + j;
+        hc = ca;
+        hm = ma;
+      }
+      ca += c[j];
+      ma += m[j];
+    }
+    if (hit < kWideBins) atomicMin(&s_bin, hit);
+    __syncthreads();
+    if (chunk == 0) {
+      if (hit < kWideBins && hit == s_bin) {
+        wr.cut->bin = hit;
+        wr.cut->c_above = hc;
+        wr.cut->m_above = hm;
+      } else if (tid == 0 && s_bin == kWideBins) {
+        wr.cut->bin = kWideBins;
+      }
+    }
+  } else {
+    // Ids of the chunks before this one.
+    uint32_t n = 0;
+    for (int c = lane; c < chunk; c += 64) n += wr.chunk_n[c];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+    if (tid == 0) {
+      s_base = (int)n;
+      s_bin = wr.cut->bin;
+    }
+    __syncthreads();
+  }
+  const int bin = s_bin;
+  bool in[kEPT], edge[kEPT];
+#pragma unroll
+  for (int e = 0; e < kEPT; ++e) {
+    const int id = chunk * kChunk + e * kSampThreads + tid;
+    const int b = wide_bin(v[e], temp, M);
+    in[e] = id < V && b <= bin;
+    edge[e] = b == bin;
+    const uint64_t bal = __ballot(in[e]);
+    if (lane == 0) s_n[e][wave] = (uint32_t)__popcll(bal);
+  }
+  __syncthreads();
+  if constexpr (!COLLECT) {
+    if (tid == 0) {
+      uint32_t n = 0;
+      for (int e = 0; e < kEPT; ++e)
+        for (int w = 0; w < NWV; ++w) n += s_n[e][w];
+      wr.chunk_n[chunk] = n;
+    }
+  } else {
+    unsigned char* rb = lawbuf + (size_t)row * row_bytes;
+    int* ids = reinterpret_cast<int*>(rb + wide_ids_off());
+    double* probs = reinterpret_cast<double*>(rb + wide_probs_off(V));
+    int at = s_base;
+#pragma unroll
+    for (int e = 0; e < kEPT; ++e) {
+      int before = 0, all = 0;
+#pragma unroll
+      for (int w = 0; w < NWV; ++w) {
+        if (w < wave) before += (int)s_n[e][w];
+        all += (int)s_n[e][w];
+      }
+      const uint64_t bal = __ballot(in[e]);
+      if (in[e]) {
+        const int pos = at + before + __popcll(bal & ((1ull << lane) - 1ull));
+        const double pv = exp((double)v[e] / temp - M) / S;
+        ids[pos] = chunk * kChunk + e * kSampThreads + tid;
+        probs[pos] = edge[e] ? -pv : pv;
+      }
+      at += all;
+    }
+  }
+}
+
+__global__ __launch_bounds__(kWideThreads) void wide_finish(const float* __restrict__ logits,
+                                                            const float* __restrict__ logits2, int nrows1,
+                                                            long long ld, int V, int n_chunks, double temp, int k_eff,
+                                                            double top_p, uint32_t* __restrict__ hist,
+                                                            unsigned char* __restrict__ lawbuf, size_t row_bytes) {
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const float* lr = wide_logits(logits, logits2, nrows1, ld, row);
+  const WideRow wr = wide_row(hist, n_chunks, row);
+  unsigned char* rb = lawbuf + (size_t)row * row_bytes;
+  WideHdr* hdr = reinterpret_cast<WideHdr*>(rb);
+  int* ids = reinterpret_cast<int*>(rb + wide_ids_off());
+  double* probs = reinterpret_cast<double*>(rb + wide_probs_off(V));
+  const WideCut cut = *wr.cut;
+  if (cut.nonfinite) {
+    if (tid == 0) {
+      hdr->n = 0;
+      hdr->nonfinite = 1;
+    }
+    return;
+  }
+  __shared__ uint32_t h_cnt[256];
+  __shared__ unsigned long long h_mass[256];
+  __shared__ uint32_t s_prefix, s_cabove, s_w[kWideWaves + 1];
+  __shared__ unsigned long long s_mabove;
+  __shared__ double s_d[kWideWaves];
+  __shared__ int s_n;
+  if (wave == 0) {
+    int n = 0;
+    for (int c = lane; c < n_chunks; c += 64) n += (int)wr.chunk_n[c];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+    if (lane == 0) {
+      s_n = n;
+      s_prefix = 0u;
+      s_cabove = cut.c_above;
+      s_mabove = cut.m_above;
+    }
+  }
+  __syncthreads();
+  const int n_in = s_n;
+  const bool all = cut.bin == kWideBins;
+  const bool nuc = top_p > 0.0 && top_p < 1.0;
+  const unsigned long long TP = nuc ? (unsigned long long)(top_p * kFix62) : ~0ull;
+  // Radix descent over the cut bin's ids (the bin holds the cut, so every pass finds its digit).
+  for (int pass = 0; pass < 4 && !all; ++pass) {
+    const int shift = 24 - 8 * pass;
+    if (tid < 256) {
+      h_cnt[tid] = 0u;
+      h_mass[tid] = 0ull;
+    }
+    __syncthreads();
+    const uint32_t prefix = s_prefix;
+    for (int i = tid; i < n_in; i += kWideThreads) {
+      const double pv = probs[i];
+      if (!signbit(pv)) continue;
+      const uint32_t key = ordered_bits(lr[ids[i]]);
+      if (pass == 0 || (key >> (shift + 8)) == prefix) {
+        const int dgt = (key >> shift) & 255;
+        atomicAdd(&h_cnt[dgt], 1u);
+        const unsigned long long P = (unsigned long long)(-pv * kFix62);
+        if (P) atomicAdd(&h_mass[dgt], P);
+      }
+    }
+    __syncthreads();
+    if (wave == 0) {   // lane l: digits 255 - 4 l .. 252 - 4 l
+      uint32_t c[4], ct = 0;
+      unsigned long long m[4], mt = 0ull;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        c[j] = h_cnt[255 - 4 * lane - j];
+        m[j] = h_mass[255 - 4 * lane - j];
+        ct += c[j];
+        mt += m[j];
+      }
+      uint32_t ci = ct;
+      unsigned long long mi = mt;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(ci, o, 64);
+        const unsigned long long z = __shfl_up(mi, o, 64);
+        if (lane >= o) {
+          ci += y;
+          mi += z;
+        }
+      }
+      uint32_t ca = s_cabove + ci - ct;
+      unsigned long long ma = s_mabove + mi - mt;
+      int sel = -1;
+      uint32_t hc = 0;
+      unsigned long long hm = 0ull;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (sel < 0 && c[j] && ((int)(ca + c[j]) >= k_eff || (nuc && ma + m[j] >= TP))) {
+          sel = 255 - 4 * lane - j;
+          hc = ca;
+          hm = ma;
+        }
+        ca += c[j];
+        ma += m[j];
+      }
+      const uint64_t bal = __ballot(sel >= 0);
+      if (bal && lane == __ffsll((unsigned long long)bal) - 1) {
+        s_prefix = (prefix << 8) | (uint32_t)sel;
+        s_cabove = hc;
+        s_mabove = hm;
+      }
+    }
+    __syncthreads();
+  }
+  // Inside the tie group (every logit equal to the cut's): members in id
+  // order, each of the same fixed-point mass Pt; the first is included.
+  const uint32_t tau = s_prefix;
+  int t_cut = 0x7fffffff;
+  if (!all) {
+    const double pt = exp((double)ordered_value(tau) / temp - cut.M) / cut.S;
+    const unsigned long long Pt = (unsigned long long)(pt * kFix62);
+    const long long t_k = (long long)k_eff - (long long)s_cabove;
+    long long t_n = 0x7fffffff;
+    if (nuc && Pt) t_n = (long long)((TP - s_mabove + Pt - 1ull) / Pt);
+    const long long t = t_k < t_n ? t_k : t_n;
+    t_cut = (int)(t < 0x7fffffff ? t : 0x7fffffff);
+  }
+  // The support, compacted in place: a tile's entries are all read before the
+  // scans' barriers, and its entries move to positions no later tile reads.
+  int out = 0, grank = 0;
+  for (int base = 0; base < n_in; base += kWideThreads) {
+    const int i = base + tid;
+    const bool valid = i < n_in;
+    const int id = valid ? ids[i] : 0;
+    const double sp = valid ? probs[i] : 0.0;
+    const bool edge = valid && signbit(sp) && !all;
+    const uint32_t key = edge ? ordered_bits(lr[id]) : 0u;
+    const bool isg = edge && key == tau;
+    int gtot = 0, gr = grank;
+    if (!all) {
+      gr += block_scan_flag(isg, s_w, &gtot);
+      grank += gtot;
+    }
+    const double pv = fabs(sp);
+    const bool keep = valid && pv > 0.0 && (!edge || key > tau || (isg && gr < t_cut));
+    int ktot;
+    const int pos = out + block_scan_flag(keep, s_w, &ktot);
+    if (keep) {
+      ids[pos] = id;
+      probs[pos] = pv;
+    }
+    out += ktot;
+  }
+  __syncthreads();
+  if (out == 0) {   // empty filter -> argmax one-hot (mtplx/sampling.py:197-199)
+    if (tid == 0) {
+      ids[0] = cut.argmax;
+      probs[0] = 1.0;
+      hdr->n = 1;
+      hdr->nonfinite = 0;
+    }
+    return;
+  }
+  // filtered / total, then the SparseDistribution renormalisation.
+  const double t1 = block_sum_f64(probs, out, s_d);
+  for (int i = tid; i < out; i += kWideThreads) probs[i] = probs[i] / t1;
+  __syncthreads();
+  const double t2 = block_sum_f64(probs, out, s_d);
+  for (int i = tid; i < out; i += kWideThreads) probs[i] = probs[i] / t2;
+  if (tid == 0) {
+    hdr->n = out;
+    hdr->nonfinite = 0;
+  }
+}
+
 // The accept loop of one request over wide laws: target rows b*(K+1)+d,
 // draft rows B*(K+1) + b*K + d; scratch: this request's residual ids/probs.
 __global__ __launch_bounds__(kWideThreads) void wide_accept_kernel(
@@ -1386,6 +1879,39 @@ MTP_API size_t mtp_sampler_workspace_bytes(int rows, int V, int top_k) {
   return n;
 }
 
+// Rows of more than two chunks build their wide laws over many workgroups; the
+// histograms live in the workspace's second half behind its ``used`` rows of
+// residual scratch. Where they don't fit (hardly any draft rows) one workgroup
+// per row builds the law.
+static uint32_t* wide_hist_area(const SamplerPlan& pl, int rows, int used, int V, unsigned char* lawbuf) {
+  const size_t rb = wide_row_bytes(V);
+  if (!pl.wide || pl.n_chunks <= 2 || (size_t)rows * wide_hist_row_words(pl.n_chunks) * 4 > (size_t)(rows - used) * rb)
+    return nullptr;
+  return reinterpret_cast<uint32_t*>(lawbuf + (size_t)(rows + used) * rb);
+}
+
+// The laws of ``rows`` rows (the first nrows1 from logits) into lawbuf.
+static int wide_laws(const float* logits, const float* logits2, int nrows1, int rows, int V, const ChunkPart* parts,
+                     const SamplerPlan& pl, double temp, double top_p, unsigned char* lawbuf, uint32_t* hist,
+                     hipStream_t st, const char* who) {
+  const size_t rb = wide_row_bytes(V);
+  const long long ld = V;
+  if (!hist) {
+    hipLaunchKernelGGL(wide_law_kernel, dim3(rows), dim3(kWideThreads), 0, st, logits, logits2, nrows1, ld, V, parts,
+                       pl.n_chunks, temp, pl.k_eff, top_p, lawbuf, rb);
+    return launch_check(who);
+  }
+  const dim3 grid(pl.n_chunks, rows), block(kSampThreads);
+  hipLaunchKernelGGL(wide_hist, grid, block, 0, st, logits, logits2, nrows1, ld, V, parts, pl.n_chunks, temp, hist);
+  hipLaunchKernelGGL(wide_collect<false>, grid, block, 0, st, logits, logits2, nrows1, ld, V, pl.n_chunks, temp,
+                     pl.k_eff, top_p, hist, lawbuf, rb);
+  hipLaunchKernelGGL(wide_collect<true>, grid, block, 0, st, logits, logits2, nrows1, ld, V, pl.n_chunks, temp,
+                     pl.k_eff, top_p, hist, lawbuf, rb);
+  hipLaunchKernelGGL(wide_finish, dim3(rows), dim3(kWideThreads), 0, st, logits, logits2, nrows1, ld, V, pl.n_chunks,
+                     temp, pl.k_eff, top_p, hist, lawbuf, rb);
+  return launch_check(who);
+}
+
 // The accept step over nt target and nd draft rows (the uniform batch has
 // nt = B (K + 1), nd = B K and null offsets).
 static int spec_accept_run(const float* target_logits, const float* draft_logits, const int32_t* draft_ids,
@@ -1413,18 +1939,18 @@ static int spec_accept_run(const float* target_logits, const float* draft_logits
   const double temp = pl.greedy ? 1.0 : temperature;
   rr.nt = nt;
   rr.nd = nd;
+  unsigned char* lawbuf = reinterpret_cast<unsigned char*>(ws) + parts_bytes(rows, V);
+  uint32_t* hist = wide_hist_area(pl, rows, B, V, lawbuf);
   // target rows then draft rows, one launch (dparts follows tparts)
   hipLaunchKernelGGL(vocab_partials, dim3(n_chunks, rows), dim3(kSampThreads), 0, st, target_logits,
                      draft_logits ? draft_logits : target_logits, nt, (long long)V, V, n_chunks, temp, pl.ksel,
-                     pl.greedy, tparts);
+                     pl.greedy, tparts, hist, hist ? (int)wide_hist_row_words(n_chunks) : 0);
   if ((rc = launch_check(who))) return rc;
   if (pl.wide) {
-    unsigned char* lawbuf = reinterpret_cast<unsigned char*>(ws) + parts_bytes(rows, V);
     const size_t rb = wide_row_bytes(V);
-    hipLaunchKernelGGL(wide_law_kernel, dim3(rows), dim3(kWideThreads), 0, st, target_logits,
-                       draft_logits ? draft_logits : target_logits, nt, (long long)V, V, tparts, n_chunks, temp,
-                       pl.k_eff, top_p, lawbuf, rb);
-    if ((rc = launch_check(who))) return rc;
+    rc = wide_laws(target_logits, draft_logits ? draft_logits : target_logits, nt, rows, V, tparts, pl, temp, top_p,
+                   lawbuf, hist, st, who);
+    if (rc) return rc;
     hipLaunchKernelGGL(wide_accept_kernel, dim3(B), dim3(kWideThreads), 0, st, lawbuf, rb, V, B, K, draft_ids,
                        uniforms, out_tokens, n_accepted, accept_probs, status, lawbuf + (size_t)rows * rb, rr);
   } else if (n_chunks <= 64) {
@@ -1564,15 +2090,16 @@ MTP_API int mtp_sample_rows(const float* logits, int rows, int V, double tempera
   hipStream_t st = (hipStream_t)stream;
   ChunkPart* parts = reinterpret_cast<ChunkPart*>(ws);
   const double temp = pl.greedy ? 1.0 : temperature;
+  unsigned char* lawbuf = reinterpret_cast<unsigned char*>(ws) + parts_bytes(rows, V);
+  uint32_t* hist = wide_hist_area(pl, rows, 0, V, lawbuf);
   hipLaunchKernelGGL(vocab_partials, dim3(pl.n_chunks, rows), dim3(kSampThreads), 0, st, logits, logits, rows,
-                     (long long)V, V, pl.n_chunks, temp, pl.ksel, pl.greedy, parts);
+                     (long long)V, V, pl.n_chunks, temp, pl.ksel, pl.greedy, parts, hist,
+                     hist ? (int)wide_hist_row_words(pl.n_chunks) : 0);
   if ((rc = launch_check(who))) return rc;
   if (pl.wide) {
-    unsigned char* lawbuf = reinterpret_cast<unsigned char*>(ws) + parts_bytes(rows, V);
     const size_t rb = wide_row_bytes(V);
-    hipLaunchKernelGGL(wide_law_kernel, dim3(rows), dim3(kWideThreads), 0, st, logits, logits, rows, (long long)V,
-                       V, parts, pl.n_chunks, temp, pl.k_eff, top_p, lawbuf, rb);
-    if ((rc = launch_check(who))) return rc;
+    rc = wide_laws(logits, logits, rows, rows, V, parts, pl, temp, top_p, lawbuf, hist, st, who);
+    if (rc) return rc;
     hipLaunchKernelGGL(wide_rows_kernel, dim3(rows), dim3(kWideThreads), 0, st, lawbuf, rb, V, uniforms, out_ids,
                        out_probs, ld_out, out_count, sampled, status);
   } else {

@@ -127,6 +127,40 @@ def test_wide_law_tie_group_cut(gpu):
             assert int(smp[r]) == S.choice(want, u[r])
 
 
+@pytest.mark.parametrize("V", [8192, 8193, 12289, 40000])   # two chunks (one workgroup per row), three and more
+@pytest.mark.parametrize("cfg", [S.SamplerConfig(0.7, 0.9, 0), S.SamplerConfig(1.0, 1.0, 0),
+                                 S.SamplerConfig(1.0, 0.97, 300), S.SamplerConfig(0.02, 0.999999, 0),
+                                 S.SamplerConfig(1.0, 0.5, 70)])
+def test_wide_law_over_many_workgroups(gpu, V, cfg):
+    """The binned wide law against the oracle: a plain row, a tie group that
+    spans chunks and straddles the cut, masked ids (-inf) and logits of the
+    type's lowest value, a flat row, one id far above the others; and a
+    non-finite row beside them, flagged alone."""
+    rng = np.random.default_rng(V)
+    logits = rng.normal(0, 3, (6, V)).astype(np.float32)
+    logits[1, 3::97] = logits[1].max() + 0.5
+    logits[2, ::2] = -np.inf
+    logits[2, 1::4] = np.finfo(np.float32).min
+    # A flat row but for one id: with all V equal, V * top_p = 36000 is a step of
+    # the nucleus itself, where the order of V sums (error <= V * 2^-53 = 5e-12)
+    # decides; the one larger id moves every step at least 1e-7 off top_p.
+    logits[3] = 0.25
+    logits[3, 7] = 0.3
+    logits[4, V - 1] = 60.0
+    logits[5, V // 2] = np.nan
+    # Off the cdf steps k / n of the flat and tied rows (equal probabilities
+    # put steps at exact fractions, where the order of the sums decides).
+    u = np.array([0.3137, 0.60713, 0.90231, 0.412137, 0.7, 0.5])
+    ids, probs, cnt, smp, st = _sample_rows(logits, cfg, u)
+    assert st.tolist() == [0, 0, 0, 0, 0, 1]
+    for r in range(5):
+        want = S.sparse_distribution(logits[r], cfg)
+        n = int(cnt[r])
+        assert ids[r, :n].tolist() == want.ids.tolist(), r
+        assert np.allclose(probs[r, :n], want.probs, rtol=0, atol=1e-9), r
+        assert int(smp[r]) == S.choice(want, u[r]), r
+
+
 def test_output_rows_use_the_given_stride(gpu):
     """Greedy with top_k = 20 (support 1) written at a row stride of 20: every
     row's slot 0 is its argmax and the rest is padded (-1, 0)."""
