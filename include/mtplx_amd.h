@@ -237,6 +237,17 @@ typedef struct mtp_qmm_args {
 size_t mtp_qmm_workspace_bytes(int M, int N, int K, int dual);
 int mtp_qmm_affine4_mfma(const mtp_qmm_args* args, void* stream);
 
+/* The same matmul for any number of rows in one launch (prompt chunks): y bf16
+ * [M, N] = x [M, K] W^T over the layout-1 pack; x 16-byte aligned, rows
+ * contiguous. ws: mtp_qmm_tiles_workspace_bytes (16-byte aligned, contents
+ * irrelevant): the group sums of x, and the K parts of small grids. Same
+ * arithmetic (dequantised weights never rounded, fp32 accumulation); a row's
+ * sums may be split by K differently from mtp_qmm_affine4_mfma's. Replaces the
+ * stock mx.quantized_matmul that mtplx/nax_verify.py:754 leaves large M to. */
+size_t mtp_qmm_tiles_workspace_bytes(int M, int N, int K);
+int mtp_qmm_affine4_tiles(const void* x, const void* w, void* y, int M, int N, int K, int group_size, void* ws,
+                          size_t ws_bytes, void* stream);
+
 /* ---- Ragged KV cache + attention -----------------------------------------
  * Cache layout [B, Hkv, cap, D] bf16 (mtplx/ragged_kv_cache.py:71).
  * Scatter: cache[b,h,write_start[b]+i,:] = new[b,h,i,:]

@@ -71,6 +71,8 @@ SIGNATURES = {
     "mtp_qmv_affine4_ex": (_i, [_vp, _vp]),
     "mtp_qmm_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "mtp_qmm_affine4_mfma": (_i, [_vp, _vp]),
+    "mtp_qmm_tiles_workspace_bytes": (_sz, [_i, _i, _i]),
+    "mtp_qmm_affine4_tiles": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _sz, _vp]),
     "mtp_attn_blocks_workspace_bytes": (_sz, [_i, _i, _i, C.c_longlong, _i]),
     "mtp_ragged_gqa_attn_blocks": (_i, [_vp, _vp]),
     "mtp_rope_qkv_to_blocks": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp, _vp]),

@@ -19,7 +19,7 @@ LIB = os.path.join(HERE, "libmtplx_amd.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["qmv.hip", "qmv_xplain.hip", "qmv_xswiglu.hip", "qmv_xpre.hip", "qmv_xrmsnorm.hip", "qmv_rope.hip",
-           "qmv_moe.hip", "qmv_generic.hip", "qmv_inplace.hip", "qmm_mfma.hip", "sampler.hip", "attention.hip", "model_ops.hip", "moe.hip"]
+           "qmv_moe.hip", "qmv_generic.hip", "qmv_inplace.hip", "qmm_mfma.hip", "qmm_tiles.hip", "sampler.hip", "attention.hip", "model_ops.hip", "moe.hip"]
 
 # Packed fp32 VALU instructions are disabled for every device pass: some
 # of their forms have produced silently wrong results on MI355X boxes of this

@@ -13,7 +13,7 @@ every fallback (:730-736). Here the patch installs the same routing on
   drop (:755-763);
 * other eligible 4-bit calls (groups 64/128, K % 256 == 0): up to 32 rows on
   the streaming verify kernel, 33..64 rows on the 9..64-row MFMA kernel over
-  the layout-1 pack, more rows in 64-row launches of it; also after the
+  the layout-1 pack, more rows on the tiles kernel over it; also after the
   layer's MLX triple has been released;
 * 8-bit layers (and 4-bit group 32) run the general affine kernel, the
   ``vk_qmm_m4`` / ``vk_qmm_m6`` lane of the reference's 8-bit branch;

@@ -16,8 +16,10 @@ Kernels, by rows M (4-bit groups of 64/128 with K % 256 == 0):
   rows and layout 1 beyond, packed once and kept like the M > 32 pack
   (cfg1 shape: 15.7 against 25.5 us for ``mtp_qmv_affine4`` on the MLX
   layout, which runs when ``MTPLX_AMD_PACK_CACHE=0``);
-* M > 32: ``mtp_qmm_affine4_mfma`` (each weight quad read once for 64 rows)
-  on the layout-1 tile-major pack, in 64-row launches. A raw MLX triple is
+* M = 33..64: ``mtp_qmm_affine4_mfma`` (each weight quad read once for 64
+  rows) on the layout-1 tile-major pack; past 64 rows ``mtp_qmm_affine4_tiles``
+  on the same pack (the greedy lane: 64-row launches, whose rows do not depend
+  on M). A raw MLX triple is
   packed once and the pack kept, keyed by the weight tensor (a verify
   forward calls every projection again each step); ``MTPLX_AMD_PACK_CACHE=0``
   packs into a temporary instead.
@@ -162,6 +164,24 @@ def rows_matmul(x2: torch.Tensor, pack: torch.Tensor, n: int, group_size: int,
     return y
 
 
+TILES_ROWS = 8192    # rows per launch of the tiles kernel (bounds its workspace)
+
+
+def tiles_matmul(x2: torch.Tensor, pack: torch.Tensor, n: int, group_size: int,
+                 out: torch.Tensor | None = None) -> torch.Tensor:
+    """``x2 [M, K] @ W.T`` on a layout-1 pack with ``mtp_qmm_affine4_tiles``:
+    what more rows than ``MFMA_ROWS`` run outside the greedy lane."""
+    m, k = (int(d) for d in x2.shape)
+    y = out if out is not None else torch.empty((m, n), dtype=torch.bfloat16, device=x2.device)
+    st = _lib.stream_handle(x2.device)
+    for r0 in range(0, m, TILES_ROWS):
+        r = min(TILES_ROWS, m - r0)
+        ws = _lib.WORKSPACES.get(_lib.query("mtp_qmm_tiles_workspace_bytes", r, n, k), "qmm_tiles", x2.device)
+        _lib.call("mtp_qmm_affine4_tiles", x2[r0:].data_ptr(), pack.data_ptr(), y[r0:].data_ptr(), r, n, k,
+                  int(group_size), ws.data_ptr(), ws.numel(), st)
+    return y
+
+
 def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, *,
                      group_size: int = 64, bits: int = 4, mode: str = "affine",
                      out: torch.Tensor | None = None, exact: bool = False) -> torch.Tensor:
@@ -177,7 +197,8 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                   None, m, n, k, group_size, bits, _lib.stream_handle(x.device))
         return y.reshape(*lead, n)
     if m > STREAM_ROWS or exact:
-        y = rows_matmul(x2, layout1_pack(w, scales, biases, group_size), n, group_size, out)
+        matmul = tiles_matmul if m > MFMA_ROWS and not exact else rows_matmul
+        y = matmul(x2, layout1_pack(w, scales, biases, group_size), n, group_size, out)
         return y.reshape(*lead, n)
     y = out if out is not None else torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     st = _lib.stream_handle(x.device)

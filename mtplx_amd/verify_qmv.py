@@ -6,7 +6,7 @@ an ineligible call returns ``module(x)`` — here the general gfx950 matmul of
 reference's fixed-M probes (M=3 "multi3", M=4 pair) are generalised to every
 verify-row count M = sum_b (K_b + 1): up to 32 rows on the streaming kernel,
 more on the 9..64-row MFMA kernel over the module's layout-1 pack (packed on
-first use and kept on the module; 64-row launches past 64 rows).
+first use and kept on the module), past 64 rows on the tiles kernel over it.
 """
 
 from __future__ import annotations
@@ -17,7 +17,8 @@ import torch
 
 from . import _lib
 from .quant import QuantizedLinear
-from .verify_kernels import STREAM_ROWS, _pack_cache_enabled, fast_path, quantized_matmul, rows_matmul
+from .verify_kernels import (MFMA_ROWS, STREAM_ROWS, _pack_cache_enabled, fast_path, quantized_matmul, rows_matmul,
+                             tiles_matmul)
 
 
 def _affine4(module: Any) -> bool:
@@ -98,7 +99,8 @@ def packed_matmul(x: torch.Tensor, module: QuantizedLinear, *, exact: bool = Fal
     GPU), or None when there is no suitable pack or x does not qualify. Up to
     32 rows stream the pack on ``mtp_qmv_affine4_ex``; more rows (or
     ``exact``: every M, the row-invariant greedy lane) run
-    ``mtp_qmm_affine4_mfma`` on the layout-1 pack. A module with an MLX
+    ``mtp_qmm_affine4_mfma`` on the layout-1 pack, past 64 rows outside the
+    greedy lane ``mtp_qmm_affine4_tiles``. A module with an MLX
     triple but no layout-1 pack gets one here when the MFMA kernel needs it.
     Never falls back to ``module(x)``, so a patched ``__call__`` may use it."""
     if len(module._shape) != 2:   # expert stacks go through switch_linear
@@ -114,7 +116,8 @@ def packed_matmul(x: torch.Tensor, module: QuantizedLinear, *, exact: bool = Fal
             if module.weight is None or not fast_path(module.bits, module.group_size, k):
                 return None
             module.pack()
-        y = rows_matmul(x2, module.packed, n, module.group_size)
+        matmul = tiles_matmul if m > MFMA_ROWS and not exact else rows_matmul
+        y = matmul(x2, module.packed, n, module.group_size)
         return _add_bias(y, module).reshape(*lead, n)
     pk = _packed(module, m)
     if pk is None:

@@ -178,3 +178,45 @@ def test_one_workspace_serves_shapes_in_turn(gpu):
         assert not torch.isnan(a.float()).any()
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
     assert int(torch.count_nonzero(ws[:65536])) == 0
+
+
+@pytest.mark.parametrize("m,n,k,gs", [
+    (65, 33, 256, 64),        # one quad; a second row tile of one row; a part of a column tile
+    (64, 128, 512, 128),      # exactly one tile
+    (127, 257, 1024, 64),     # two quads in K parts (16 workgroups)
+    (200, 1000, 2816, 64),    # 11 quads over K parts of unequal length
+    (130, 5120, 512, 64),     # 120 workgroups of two quads
+    (193, 8224, 768, 128),    # more workgroups than CUs: no K parts
+    (65, 4096, 12288, 64),    # 48 quads
+])
+def test_tiles_match_oracle(gpu, m, n, k, gs):
+    """mtp_qmm_affine4_tiles at the edges of its row tiles (64), column groups
+    (128) and K parts; no row past the last is written, and a NaN row stays
+    in its own row."""
+    from mtplx_amd import _lib
+    from mtplx_amd.quant import QuantizedLinear
+    from oracle.qmv import make_affine4_weights
+    from tests.gpu_util import from_bits, randn_bf16, u32
+    rng = np.random.default_rng(m + n + k)
+    w, s, bb = make_affine4_weights(rng, n, k, gs)
+    q = QuantizedLinear(u32(w), from_bits(s), from_bits(bb), group_size=gs)
+    x = randn_bf16(rng, (m, k))
+    y = torch.full((m + 1, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    pack = q.pack()
+    ws = torch.full((_lib.query("mtp_qmm_tiles_workspace_bytes", m, n, k),), 255, dtype=torch.uint8, device="cuda")
+    args = (pack.data_ptr(), y.data_ptr(), m, n, k, gs, ws.data_ptr(), ws.numel(),
+            torch.cuda.current_stream().cuda_stream)
+    _lib.call("mtp_qmm_affine4_tiles", x.data_ptr(), *args)
+    torch.cuda.synchronize()
+    assert torch.isnan(y[m]).all()
+    want = round_to_bf16(qmm_affine4(bits(x), w, s, bb, gs))
+    assert_close(bf16_values(y[:m]), want, what=f"tiles m={m} n={n} k={k}")
+    first = y[:m].clone()
+    x[m // 2, k - 1] = float("nan")
+    _lib.call("mtp_qmm_affine4_tiles", x.data_ptr(), *args)
+    torch.cuda.synchronize()
+    keep = torch.arange(m) != m // 2
+    assert torch.isnan(y[m // 2]).all() and torch.equal(y[:m][keep], first[keep])
+    # a workspace one byte short is refused
+    with pytest.raises(_lib.MtpError):
+        _lib.call("mtp_qmm_affine4_tiles", x.data_ptr(), *args[:-2], ws.numel() - 1, args[-1])
