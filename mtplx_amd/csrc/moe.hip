@@ -303,22 +303,36 @@ __global__ __launch_bounds__(kSortThreads) void moe_segments_kernel(const int32_
     if (tid == 0) active[0] = -1;
     return;
   }
-  // off[e] = first i with sorted_ids[i] >= e (binary search per expert).
-  for (int e = tid; e <= E; e += kSortThreads) {
-    int lo = 0, hi = R;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (sorted_ids[mid] < e) lo = mid + 1; else hi = mid;
+  // A row that starts an expert's run writes the offsets of that expert and of
+  // the empty ones before it, and the expert's place in the active list (the
+  // runs before it: ballots and the waves' counts, 1024 rows a round). 26 us ->
+  // 3 for 128 rows of 256 experts, 40 -> 7 for 4096, against a binary search
+  // per expert and one thread listing the experts.
+  __shared__ int s_w[kSortThreads / 64];
+  const int lane = tid & 63, wave = tid >> 6;
+  int na = 0;
+  for (int c0 = 0; c0 < R; c0 += kSortThreads) {
+    const int i = c0 + tid;
+    const int e = i < R ? sorted_ids[i] : 0;
+    const int prev = i > 0 && i < R ? sorted_ids[i - 1] : -1;
+    const bool first = i < R && e != prev;
+    const unsigned long long bal = __ballot(first);
+    if (lane == 0) s_w[wave] = __popcll(bal);
+    __syncthreads();
+    int at = na + __popcll(bal & ((1ull << lane) - 1ull));
+    for (int w = 0; w < kSortThreads / 64; ++w) {
+      if (w < wave) at += s_w[w];
+      na += s_w[w];
     }
-    expert_off[e] = lo;
+    if (first) {
+      active[1 + at] = e;
+      for (int f = prev + 1; f <= e; ++f) expert_off[f] = i;
+    }
+    if (i == R - 1)
+      for (int f = e + 1; f <= E; ++f) expert_off[f] = R;
+    __syncthreads();   // s_w is rewritten by the next round
   }
-  __syncthreads();
-  if (tid == 0) {
-    int na = 0;
-    for (int e = 0; e < E; ++e)
-      if (expert_off[e + 1] > expert_off[e]) active[1 + na++] = e;
-    active[0] = na;
-  }
+  if (tid == 0) active[0] = na;
 }
 
 }  // namespace mtp

@@ -81,6 +81,20 @@ def test_segments_from_sorted_ids(gpu):
     assert int(act[0]) == -1
 
 
+@pytest.mark.parametrize("R,E,lo,hi", [(1, 1, 0, 1), (1, 600, 599, 600), (1024, 64, 0, 64), (1025, 300, 40, 200),
+                                       (5000, 4096, 3, 4090), (2048, 8, 7, 8)])
+def test_segments_over_rounds(gpu, R, E, lo, hi):
+    """Offsets and active list over several rounds of 1024 rows, with empty
+    experts before, between and after."""
+    from mtplx_amd.moe_sorted_gather import segments
+    rng = np.random.default_rng(R + E)
+    ids = np.sort(rng.integers(lo, hi, size=R)).astype(np.int32)
+    off, act = segments(torch.from_numpy(ids).cuda(), E)
+    assert off.cpu().numpy().tolist() == np.searchsorted(ids, np.arange(E + 1)).tolist()
+    a, want = act.cpu().numpy(), np.unique(ids).tolist()
+    assert a[0] == len(want) and a[1:1 + a[0]].tolist() == want
+
+
 def _experts(rng, E, H, F):
     gu = make_affine4_weights(rng, E * 2 * F, H)
     gu = tuple(a.reshape(E, 2 * F, -1) for a in gu)
