@@ -65,9 +65,10 @@ static void inplace_rows(InplaceParams p, int max_rows, hipStream_t st) {
 template <int BITS, int GS, bool DUAL>
 static void inplace_vec(const InplaceParams& p, int max_rows, hipStream_t st) {
   // Scales straight to LDS in 16-byte pieces of eight groups where rows hold
-  // whole pieces and the arrays are so aligned; else element by element.
+  // whole pieces and the arrays are so aligned; else element by element. x may
+  // start at any element too.
   auto aligned = [](const void* a) { return ((uintptr_t)a & 15) == 0; };
-  const bool vec = (p.K / GS) % 8 == 0 && aligned(p.s0) && aligned(p.b0) &&
+  const bool vec = (p.K / GS) % 8 == 0 && aligned(p.x) && aligned(p.s0) && aligned(p.b0) &&
                    (!DUAL || (aligned(p.s1) && aligned(p.b1)));
   if (vec) {
     inplace_rows<BITS, GS, DUAL, true>(p, max_rows, st);

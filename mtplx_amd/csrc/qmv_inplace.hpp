@@ -117,7 +117,8 @@ __device__ __forceinline__ void group_vals(const unsigned char* at, float (&o)[G
   for (int u = 0; u < GPC; ++u) o[u] = __uint_as_float((u & 1) ? (v[u >> 1] & 0xffff0000u) : (v[u >> 1] << 16));
 }
 
-// VEC: scales straight to LDS (else element by element). XS: the bias term
+// VEC: scales straight to LDS, and x 16-byte aligned (else scales element by
+// element, and x too where it is not aligned). XS: the bias term
 // takes its group sums from the caller's chunk-sum table (p.xsums).
 template <int BITS, int GS, int R, bool DUAL, bool VEC, bool XS, int NW, int KS, int ND>
 __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
@@ -145,6 +146,7 @@ __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
   const int Q = (p.K + S::CK - 1) / S::CK;
   const bool tail_k = (p.K % S::CK) != 0;
   const int sgroups = p.K / GS;
+  const bool x_al = ((uintptr_t)p.x & 15) == 0;   // (rows are whole 64-byte steps apart)
   unsigned char* const stage0 = smem + (size_t)wave * S::D * S::STAGE;
   const uint32_t lds0 = lds_addr(stage0);
   float* const red = reinterpret_cast<float*>(smem + (size_t)NW * S::D * S::STAGE);
@@ -382,7 +384,16 @@ __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
           const int r = i * (64 / LPR) + x_r;
           int k = S::CK * q + 8 * (x_slot ^ (r & 15));
           if (tail_k && k >= p.K) k = 0;
-          dma16(x_ptr[i] + k, st + COLS * 128 + 1024 * i);
+          if (VEC || x_al) {
+            dma16(x_ptr[i] + k, st + COLS * 128 + 1024 * i);
+          } else {   // x at any element: the wave waits for it, and so for all loads before it
+            uint32_t v[4];
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+              v[h] = x_ptr[i][k + 2 * h] | (uint32_t)x_ptr[i][k + 2 * h + 1] << 16;
+            *reinterpret_cast<uint4*>(stage0 + (st - lds0) + COLS * 128 + 1024 * i + 16 * lane) =
+                make_uint4(v[0], v[1], v[2], v[3]);
+          }
         }
         ++pf_t;
         advance();

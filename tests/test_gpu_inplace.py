@@ -40,6 +40,28 @@ def test_tile_edges(gpu, b, gs, n, k, m):
     assert_close(bf16_values(y[:m]), round_to_bf16(qmm_affine(bits(x), w, s, bb, gs, b)), what="in place")
 
 
+@pytest.mark.parametrize("b,gs,k", [(4, 32, 288), (8, 64, 1024), (8, 128, 5120)])
+@pytest.mark.parametrize("m", [1, 4, 5, 17])
+def test_rows_at_any_alignment(gpu, b, gs, k, m):
+    """x that starts 2 bytes into an allocation: the same outputs (the same
+    products and sums: only the way x reaches LDS differs)."""
+    from mtplx_amd import _lib
+    rng = np.random.default_rng(6)
+    n = 97
+    w, s, bb = make_affine_weights(rng, n, k, gs, b)
+    x, wd, sd, bd = randn_bf16(rng, (m, k)), u32(w), from_bits(s), from_bits(bb)
+    xo = torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].reshape(m, k)
+    assert xo.data_ptr() % 16 == 2
+    ys = []
+    for x_ in (x, xo):
+        y = torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
+        _lib.call("mtp_qmv_affine", x_.data_ptr(), wd.data_ptr(), sd.data_ptr(), bd.data_ptr(), y.data_ptr(), None, m,
+                  n, k, gs, b, torch.cuda.current_stream().cuda_stream)
+        ys.append(y)
+    torch.cuda.synchronize()
+    assert torch.equal(ys[0], ys[1])
+
+
 def test_scales_at_any_alignment(gpu):
     """Scale arrays that start 2 bytes into an allocation: the same outputs."""
     from mtplx_amd import _lib
