@@ -11,9 +11,9 @@ static void inplace_run(InplaceParams p, hipStream_t st) {
   using S = InplaceShape<BITS, GS, R, DUAL, NW, KS, ND>;
   auto k = qmv_inplace_kernel<BITS, GS, R, DUAL, VEC, XS, NW, KS, ND>;
   constexpr int lds = (int)S::lds();
-  // Workgroups per CU by LDS (static part: under 5 KB), at most two.
-  constexpr int per_cu = 160 * 1024 / (lds + 5120) >= 2 ? 2 : 1;
-  static_assert(lds + 5120 <= 160 * 1024, "a workgroup's LDS");
+  // Workgroups per CU by LDS, at most two.
+  constexpr int per_cu = 160 * 1024 / (lds + S::FIXED) >= 2 ? 2 : 1;
+  static_assert(lds + S::FIXED <= 160 * 1024, "a workgroup's LDS");
   (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   p.ntile = cdiv(p.N, S::OC);
   int grid = per_cu * device_cus();

@@ -17,7 +17,7 @@
 //    or two column groups, between them) and meet once per item (column tile
 //    x row tile), their sums added in wave order;
 //  * scales and biases of an item's columns come as whole rows, also straight
-//    to LDS (up to 88 groups of a row at a time), an item ahead: fetched chunk
+//    to LDS (up to 88 or 24 groups of a row at a time), an item ahead: fetched chunk
 //    by chunk, every 4 bytes of them cost a cache line (8-bit, 32768 x 5120,
 //    4 rows: 41.2 us against 36.1);
 //  * 16-byte pieces of a line sit at slot piece ^ (row / 2 % 8), those of an x
@@ -70,16 +70,20 @@ struct InplaceParams {
 };
 
 constexpr int kInList = 128;    // experts listed in LDS at a time
-constexpr int kInItems = 32;    // items described in LDS at a time
-// Scale groups of one column staged at a time: a longer K takes its groups in
-// several segments. An LDS row is an odd number of 16-byte pieces, so 16
-// columns' reads fall in distinct banks.
-constexpr int kInGroups = 88;
-constexpr int kInSRow = 16 * 11;
-
 template <int BITS, int GS, int R, bool DUAL, int NW, int KS, int ND>
 struct InplaceShape {
   static constexpr int D = ND;                      // stages per wave
+  // Scale groups of one column staged at a time: a longer K takes its groups in
+  // several segments. An LDS row is an odd number of 16-byte pieces, so 16
+  // columns' reads fall in distinct banks. The experts' tiles of 16 rows stage
+  // few groups and items, so that two workgroups (81 KB each) fit a CU, at
+  // most 256 registers: their waves' own instructions bound them, and one wave
+  // per SIMD leaves every wait open (256 experts of 1536 x 4096, 512 rows x 8:
+  // 1366 us with 88 groups and one workgroup per CU, 1014 with 24 and two).
+  static constexpr bool SMALL = R == 16 && ND == 1;
+  static constexpr int GRP = SMALL ? 24 : 88;
+  static constexpr int SROW = 2 * GRP;
+  static constexpr int ITEMS = SMALL ? 16 : 32;     // items described in LDS at a time
   static constexpr int COLS = 32;                   // weight rows per wave
   static constexpr int CK = 1024 / BITS;            // k per chunk
   static constexpr int XB = CK * 2;                 // x bytes per row and chunk
@@ -88,13 +92,15 @@ struct InplaceShape {
   static constexpr int XI = XR * XB / 1024;         // x load instructions per chunk
   static constexpr int WI = COLS / 8;               // weight load instructions per chunk
   static constexpr int STAGE = COLS * 128 + XR * XB;
-  static constexpr int SEG = kInGroups / GPC;         // chunks per scale segment
+  static constexpr int SEG = GRP / GPC;         // chunks per scale segment
   static constexpr int TC = COLS * (NW / KS);         // weight rows per tile
   static constexpr int OC = DUAL ? TC / 2 : TC;       // output columns per tile
-  static constexpr int SCAL = 2 * TC * kInSRow;       // one segment: scales [TC][row], then biases
+  static constexpr int SCAL = 2 * TC * SROW;       // one segment: scales [TC][row], then biases
   static constexpr int RED = 2 * NW * XR * COLS * 4;
   static constexpr size_t lds() { return (size_t)NW * D * STAGE + RED + 2 * SCAL; }
-  static_assert(kInGroups % GPC == 0 && kInGroups % 8 == 0, "segments of whole chunks and 16-byte pieces");
+  static_assert(GRP % GPC == 0 && GRP % 8 == 0, "segments of whole chunks and 16-byte pieces");
+  static constexpr int FIXED = 2 * kInList * 4 + (kInList + 1) * 4 + 8 * NW + ITEMS * (16 + 4 * XR) + 64;   // static LDS
+  static_assert((GRP / 8) % 2 == 1, "odd rows");
   static_assert(XI >= 1, "a chunk of x is at least one load");
 };
 
@@ -121,7 +127,7 @@ __device__ __forceinline__ void group_vals(const unsigned char* at, float (&o)[G
 // element, and x too where it is not aligned). XS: the bias term
 // takes its group sums from the caller's chunk-sum table (p.xsums).
 template <int BITS, int GS, int R, bool DUAL, bool VEC, bool XS, int NW, int KS, int ND>
-__global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
+__global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inplace_kernel(InplaceParams p) {
   using S = InplaceShape<BITS, GS, R, DUAL, NW, KS, ND>;
   constexpr int COLS = S::COLS;
   static_assert(!DUAL || NW == 2 * KS, "the pair: half the waves on each matrix");
@@ -134,8 +140,8 @@ __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_e[kInList], s_r0[kInList], s_cum[kInList + 1];
   __shared__ int s_wcnt[NW], s_wtil[NW];
-  __shared__ int4 s_item[kInItems];          // expert, column tile, first row, rows
-  __shared__ int s_rows[kInItems][S::XR];    // x row of each staged row
+  __shared__ int4 s_item[S::ITEMS];          // expert, column tile, first row, rows
+  __shared__ int s_rows[S::ITEMS][S::XR];    // x row of each staged row
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -167,7 +173,7 @@ __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
 
   // Scales: wave instruction i loads pieces 64 i .. + 63 of the buffer, piece
   // pc of row r (a column's scales, or its biases) at r * PR + pc.
-  constexpr int PR = kInSRow / 16;
+  constexpr int PR = S::SROW / 16;
   constexpr int NI = 2 * S::TC * PR / 64;
   constexpr int NJ = (NI + NW - 1) / NW;
   static_assert(2 * S::TC * PR % 64 == 0, "whole wave instructions");
@@ -253,10 +259,10 @@ __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
     __syncthreads();
     const int n_items = s_cum[n_list] * p.ntile;
 
-    // This workgroup's items blockIdx.x, + gridDim.x, ..., kInItems at a time.
-    for (int i0 = blockIdx.x; i0 < n_items; i0 += kInItems * gridDim.x) {
+    // This workgroup's items blockIdx.x, + gridDim.x, ..., S::ITEMS at a time.
+    for (int i0 = blockIdx.x; i0 < n_items; i0 += S::ITEMS * gridDim.x) {
       const int left = (n_items - i0 + (int)gridDim.x - 1) / (int)gridDim.x;
-      const int ni = left < kInItems ? left : kInItems;
+      const int ni = left < S::ITEMS ? left : S::ITEMS;
       __syncthreads();   // the last items' readers are done
       for (int j = tid; j < ni * S::XR; j += NT) {
         const int it = j / S::XR, r = j - it * S::XR;
@@ -306,8 +312,8 @@ __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
       auto load_scales = [&](int it, int sg) {
         const int4 im = s_item[it];
         const int n0 = im.y * S::OC;
-        const int g0 = sg * kInGroups;
-        const int ng = sgroups - g0 < kInGroups ? sgroups - g0 : kInGroups;
+        const int g0 = sg * S::GRP;
+        const int ng = sgroups - g0 < S::GRP ? sgroups - g0 : S::GRP;
         const int buf = ((it * nseg + sg) & 1) * S::SCAL;
         const size_t eo = (size_t)(im.x * p.s_estride) + g0;
         if constexpr (VEC) {
@@ -325,14 +331,14 @@ __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
           }
         } else {
           // (groups past K, of a last chunk that is not whole, as zero)
-          const int np = S::GPC * Q - g0 < kInGroups ? S::GPC * Q - g0 : kInGroups;
+          const int np = S::GPC * Q - g0 < S::GRP ? S::GPC * Q - g0 : S::GRP;
           for (int t = tid; t < 2 * S::TC * np; t += NT) {
             const int row = t / np, u = t - row * np;
             const int c = row % S::TC;
             const int col = n0 + (DUAL ? c % S::OC : c);
             const bool up = DUAL && c >= S::OC;
             const uint16_t* const src = row >= S::TC ? (up ? p.b1 : p.b0) : (up ? p.s1 : p.s0);
-            *reinterpret_cast<uint16_t*>(scal + buf + row * kInSRow + 2 * u) =
+            *reinterpret_cast<uint16_t*>(scal + buf + row * S::SROW + 2 * u) =
                 u < ng ? src[eo + (size_t)(col < p.N ? col : p.N - 1) * sgroups + u] : (uint16_t)0;
           }
         }
@@ -449,9 +455,9 @@ __global__ __launch_bounds__(NW * 64) void qmv_inplace_kernel(InplaceParams p) {
         const int g0 = (q - sg * S::SEG) * S::GPC;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-          const unsigned char* const sp = sc + (COLS * cg + 16 * ct + c16) * kInSRow + 2 * g0;
+          const unsigned char* const sp = sc + (COLS * cg + 16 * ct + c16) * S::SROW + 2 * g0;
           group_vals<S::GPC>(sp, o.s[ct]);
-          group_vals<S::GPC>(sp + S::TC * kInSRow, o.b[ct]);
+          group_vals<S::GPC>(sp + S::TC * S::SROW, o.b[ct]);
         }
       };
       auto compute = [&](const Ops& o, int q) {

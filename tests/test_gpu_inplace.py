@@ -86,6 +86,10 @@ def test_scales_at_any_alignment(gpu):
     (4, 70, 4, 512, 64, 128, 0.0),      # 70 rows each: five row tiles
     (160, 40, 8, 768, 4128, 64, 1.5),   # more items per workgroup than one list (32), both row classes
     (3, 9, 1, 1536, 40, 64, 0.0),       # columns past a tile; K in 6 chunks over 2 waves
+    # tiles of 16 rows, scales in segments of 24 groups: 2 of them, the last one chunk of
+    # one wave's (28 groups); 32; 3 (60); 2 of 12 chunks (32 groups of 128)
+    (3, 40, 2, 1792, 40, 64, 0.0), (5, 60, 3, 2048, 48, 64, 0.8), (3, 40, 2, 3840, 33, 64, 0.0),
+    (3, 40, 2, 4096, 40, 128, 0.0),
 ])
 def test_experts(gpu, E, T, k, H, F, gs, skew):
     from mtplx_amd import _lib
