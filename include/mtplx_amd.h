@@ -53,12 +53,14 @@ int mtp_qmv_affine4(const void* x, const void* w, const void* scales, const void
  * q|k|v projection can write RoPE'd rows and the K/V cache itself. */
 int mtp_qmv_rope_fusable(int M, int N, int K);
 
-/* General affine quantized matmul for the formats the MFMA kernel does not
- * take: bits 4 or 8, group_size 32, 64 or 128, any M >= 1 (launches of 8
- * rows), K a multiple of 32 and of group_size, w 16-byte aligned. Weights
- * uint32 [N, K*bits/32] (little-endian bit fields), scales/biases bf16
- * [N, K/gs]; x bf16 [M, K]; output bf16 y or (y NULL) fp32 yf holding bf16
- * values, [M, N]. fp32 accumulation, VALU (not the HBM-rate lane).
+/* General affine quantized matmul for the formats that have no tile-major
+ * pack: bits 4 or 8, group_size 32, 64 or 128, any M >= 1 in one launch
+ * (tiles of 4 or 16 rows), K a multiple of 32 and of group_size, w 16-byte
+ * aligned. Weights uint32 [N, K*bits/32] (little-endian bit fields), read in
+ * place, scales/biases bf16 [N, K/gs]; x bf16 [M, K]; output bf16 y or (y
+ * NULL) fp32 yf holding bf16 values, [M, N]. bf16 MFMA on exact fields, fp32
+ * accumulation. A row's sums run in an order fixed by (K, bits, group_size):
+ * its output has the same bits for every M and whatever the other rows are.
  * Replaces: mtplx/verify_qmv.py:1377 stocklike_qmv8_matmul (8-bit verify
  * rows, eligibility :1256), the group-32 routes of
  * mtplx/kernels/qmv4_matmul.py:185 qmv4_matmul and

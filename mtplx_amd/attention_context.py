@@ -7,10 +7,11 @@ that a greedy verify picks the same argmax as autoregressive decode, and its
 operator patch then drops to one stock matmul (``mtplx/nax_verify.py:755``).
 
 Here the greedy lane is the *exact lane*: every projection runs on the
-9..64-row MFMA matmul, whose K split is planned from (N, K, CUs) alone, and
-attention runs a fixed split length with the per-head merge, so each row's
-arithmetic is the same at M = 1, at M = 4 and inside a ragged batch
-(bit-identical logits). The reference arms its guard only under
+9..64-row MFMA matmul, whose K split is planned from (N, K, CUs) alone (the
+formats without a tile-major pack on the in-place matmul, whose K split is
+the same for every M), and attention runs a fixed split length with the
+per-head merge, so each row's arithmetic is the same at M = 1, at M = 4 and
+inside a ragged batch (bit-identical logits). The reference arms its guard only under
 ``MTPLX_EXACT_T0_GUARD=1`` because its stock kernels still flip across M;
 this build's lane keeps the promise, so the guard is armed by default and
 ``MTPLX_EXACT_T0_GUARD=0`` disarms it.

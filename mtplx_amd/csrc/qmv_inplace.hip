@@ -24,7 +24,8 @@ static void inplace_run(InplaceParams p, hipStream_t st) {
   hipLaunchKernelGGL(k, dim3(grid), dim3(NW * 64), lds, st, p);
 }
 
-// One matrix: 32 columns a workgroup, K split over all of its waves. Up to 4
+// One matrix: 32 columns a workgroup, K split over all of its waves, in the
+// same eight parts for any number of rows. Up to 4
 // rows, 8 waves and two stages (17408 x 5120 of 8 bits 24.2 us, 5120 x 17408
 // 23.9; two workgroups of 4 waves 23.8 and 27.1, with one stage 25.8 and
 // 33.3); more rows, 4 waves, whose stages hold 16 rows of x (32768 x 5120, 16

@@ -15,7 +15,13 @@
 //    operands go to registers and it is loaded again while they are computed
 //    on. The waves of a workgroup split K by chunks (and the pair's matrices,
 //    or two column groups, between them) and meet once per item (column tile
-//    x row tile), their sums added in wave order;
+//    x row tile). One matrix has eight K parts whatever its rows: eight waves
+//    with one each, or four with two (chunks of the one and of the other in
+//    turn), and parts w and w + 4 are added before the four such sums are, in
+//    order of w. So a row's output has the same bits whatever rows are beside
+//    it (16 rows of 17408 x 5120, 8 bits, weights in the caches: 26.5 us; with
+//    four parts in all, one per wave, 26.1, and other bits than the eight of
+//    up to 4 rows). The experts have two parts;
 //  * scales and biases of an item's columns come as whole rows, also straight
 //    to LDS (up to 88 or 24 groups of a row at a time), an item ahead: fetched chunk
 //    by chunk, every 4 bytes of them cost a cache line (8-bit, 32768 x 5120,
@@ -73,6 +79,9 @@ constexpr int kInList = 128;    // experts listed in LDS at a time
 template <int BITS, int GS, int R, bool DUAL, int NW, int KS, int ND>
 struct InplaceShape {
   static constexpr int D = ND;                      // stages per wave
+  static constexpr int KP = KS == 2 ? 2 : 8;        // K parts: chunk c of a scale segment is in part c % KP
+  static constexpr int PW = KP / KS;                // parts per wave: its chunks take them in turn
+  static_assert(KP % KS == 0 && PW <= 2, "one or two parts per wave");
   // Scale groups of one column staged at a time: a longer K takes its groups in
   // several segments. An LDS row is an odd number of 16-byte pieces, so 16
   // columns' reads fall in distinct banks. The experts' tiles of 16 rows stage
@@ -405,11 +414,14 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
         advance();
       };
 
-      float acc[CT][RA];
+      // Sums of the wave's K parts.
+      float acc[S::PW][CT][RA];
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
+      for (int h = 0; h < S::PW; ++h)
 #pragma unroll
-        for (int i = 0; i < RA; ++i) acc[ct][i] = 0.f;
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int i = 0; i < RA; ++i) acc[h][ct][i] = 0.f;
 
       // Operands of one chunk in registers: the stage can be loaded again while
       // they are computed on.
@@ -460,7 +472,7 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
           group_vals<S::GPC>(sp + S::TC * S::SROW, o.b[ct]);
         }
       };
-      auto compute = [&](const Ops& o, int q) {
+      auto compute = [&](const Ops& o, int q, float (&acc)[CT][RA]) {
         const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 #pragma unroll
         for (int u = 0; u < S::GPC; ++u) {
@@ -517,15 +529,17 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
             const float cf = BITS == 4 ? fmaf(-128.f, o.s[ct][u], XS ? 0.f : o.b[ct][u]) : o.b[ct][u];
 #pragma unroll
             for (int i = 0; i < RA; ++i) {
-              if constexpr (XS) acc[ct][i] = fmaf(o.b[ct][u], T[i], acc[ct][i]);
-              acc[ct][i] = fmaf(o.s[ct][u], G[i], fmaf(cf, X[i], acc[ct][i]));
+              float& t = acc[ct][i];
+              if constexpr (XS) t = fmaf(o.b[ct][u], T[i], t);
+              t = fmaf(o.s[ct][u], G[i], fmaf(cf, X[i], t));
             }
           }
         }
       };
 
       // End of item it: the waves' sums meet in LDS (two areas in turn, so one
-      // barrier per item suffices), added in wave order, then stored.
+      // barrier per item suffices), added in wave order (eight parts: w and
+      // w + 4 first), then stored.
       auto finish = [&](int it) {
         float* const rd = red + (size_t)(it & 1) * NW * S::XR * COLS;
         float* const mine = rd + (size_t)wave * S::XR * COLS;
@@ -534,8 +548,9 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
 #pragma unroll
           for (int i = 0; i < RA; ++i) {
             const int m = R == 4 ? g : 4 * g + i;
-            mine[m * COLS + 16 * ct + c16] = acc[ct][i];
-            acc[ct][i] = 0.f;
+            mine[m * COLS + 16 * ct + c16] = S::PW == 2 ? acc[0][ct][i] + acc[S::PW - 1][ct][i] : acc[0][ct][i];
+#pragma unroll
+            for (int h = 0; h < S::PW; ++h) acc[h][ct][i] = 0.f;
           }
         lds_barrier();
         const int4 im = s_item[it];
@@ -544,9 +559,10 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
           const int col = im.y * S::OC + c;
           if (m >= im.w || col >= p.N) continue;
           auto sum = [&](int cc) {   // column cc of the tile's weight rows
+            auto part = [&](int w) { return rd[((cc / COLS * KS + w) * S::XR + m) * COLS + cc % COLS]; };
             float t = 0.f;
 #pragma unroll
-            for (int w = 0; w < KS; ++w) t += rd[((cc / COLS * KS + w) * S::XR + m) * COLS + cc % COLS];
+            for (int w = 0; w < (KS == 8 ? 4 : KS); ++w) t += KS == 8 ? part(w) + part(w + 4) : part(w);
             return t;
           };
           const float v = sum(c), up = DUAL ? sum(S::OC + c) : 0.f;
@@ -585,15 +601,21 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
         for (int sg = 0; sg < nseg; ++sg) {
           const unsigned char* const sc = scal + ((it * nseg + sg) & 1) * S::SCAL;
           const int n = any ? seg_chunks(sg) : 0;
-          for (int t = 0; t < n; ++t) {
+          auto chunk = [&](int t, float (&acc)[CT][RA]) {
             wait_vm<(S::D - 1) * NL>();   // the other stages' loads may be in flight
             const int q = sg * S::SEG + kw + KS * t;
             Ops o;
             fetch(o, stage0 + sel * S::STAGE, sc, sg, q);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // its reads have returned: load it again
             issue(lds0 + sel * S::STAGE);
-            compute(o, q);
+            compute(o, q, acc);
             sel = sel + 1 == S::D ? 0 : sel + 1;
+          };
+          for (int t = 0; t < n; t += S::PW) {
+            chunk(t, acc[0]);
+            if constexpr (S::PW == 2) {
+              if (t + 1 < n) chunk(t + 1, acc[1]);
+            }
           }
           // Its part of the next segment's scales: complete by the second chunk's
           // wait; with fewer chunks, waited for here.

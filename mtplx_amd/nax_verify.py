@@ -16,7 +16,8 @@ every fallback (:730-736). Here the patch installs the same routing on
   the layout-1 pack, more rows on the tiles kernel over it; also after the
   layer's MLX triple has been released;
 * 8-bit layers (and 4-bit group 32) run the general affine kernel, the
-  ``vk_qmm_m4`` / ``vk_qmm_m6`` lane of the reference's 8-bit branch;
+  ``vk_qmm_m4`` / ``vk_qmm_m6`` lane of the reference's 8-bit branch, inside
+  ``exact_verify(True)`` too (a row's bits there do not depend on M);
 * anything else falls through to the original call and is counted.
 """
 

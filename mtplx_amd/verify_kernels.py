@@ -25,7 +25,8 @@ Kernels, by rows M (4-bit groups of 64/128 with K % 256 == 0):
   packs into a temporary instead.
 
 Other MLX affine packs (4- or 8-bit, groups 32/64/128, K % 32 == 0) take
-``mtp_qmv_affine`` (``csrc/qmv_generic.hip``). There is no CPU path.
+``mtp_qmv_affine`` (``csrc/qmv_generic.hip``, on the in-place matmul of
+``csrc/qmv_inplace.hpp``). There is no CPU path.
 
 The fixed-M names keep the reference's signatures and eligibility ranges
 (4 rows; 5..6 rows), widened to the formats these kernels take; every
@@ -186,7 +187,8 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                      group_size: int = 64, bits: int = 4, mode: str = "affine",
                      out: torch.Tensor | None = None, exact: bool = False) -> torch.Tensor:
     """``x @ dequantize(w, scales, biases).T`` for ``x`` of shape ``[..., K]``.
-    ``exact``: every M on the row-invariant MFMA kernel (the greedy lane)."""
+    ``exact``: every M on the row-invariant MFMA kernel (the greedy lane);
+    the general formats' kernel is row-invariant as it is."""
     n, k = _check(x, w, scales, biases, group_size, bits, mode)
     lead = x.shape[:-1]
     x2 = x.reshape(-1, k).contiguous()

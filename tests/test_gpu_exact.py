@@ -135,3 +135,34 @@ def test_greedy_logits_bit_identical_across_batches(gpu):
     vc = [vstd[li][None].float().cpu().numpy().astype(np.float64) for li in range(cfg.layers)]
     want = verify_forward(model_params_numpy(model), cfg, toks_r[None].cpu().numpy(), np.array([qs_r]), kc, vc)
     assert_close(l4.cpu().numpy().astype(np.float64), want, what="exact lane logits")
+
+
+@pytest.mark.parametrize("b,gs,n,k", [
+    (8, 64, 2048, 5120), (8, 128, 1056, 12288), (8, 32, 1040, 5696), (4, 32, 2048, 5120),
+    (4, 64, 1024, 5184), (4, 128, 1024, 5248),   # K % 256 != 0: a last chunk that is not whole
+])
+def test_general_formats_do_not_depend_on_the_batch(gpu, b, gs, n, k):
+    """The formats without a tile-major pack (a mixed pack's 8-bit layers,
+    group 32, K % 256 != 0) inside ``exact_verify(True)``: each row's output
+    has the same bits alone, among one request's rows and in a batch."""
+    from mtplx_amd.attention_context import exact_verify
+    from mtplx_amd.nax_verify import install_nax_qlinear_patch, uninstall_nax_qlinear_patch
+    from mtplx_amd.quant import QuantizedLinear
+    from oracle.qmv import make_affine_weights
+    from tests.gpu_util import from_bits, randn_bf16, u32
+    rng = np.random.default_rng(b + gs + n + k)
+    w, s, bb = make_affine_weights(rng, n, k, gs, b)
+    layer = QuantizedLinear(u32(w), from_bits(s), from_bits(bb), group_size=gs, bits=b)
+    x = randn_bf16(rng, (45, k))
+    install_nax_qlinear_patch()
+    try:
+        with exact_verify(True):
+            want = layer(x)
+            for m in (1, 4, 5, 8, 16, 17, 33):
+                got = layer(x[:m])
+                assert torch.equal(got.view(torch.int16), want[:m].view(torch.int16)), f"rows differ at M={m} and M=45"
+            for r in (7, 20, 44):
+                got = layer(x[r:r + 1])
+                assert torch.equal(got.view(torch.int16), want[r:r + 1].view(torch.int16)), f"row {r} differs alone"
+    finally:
+        uninstall_nax_qlinear_patch()
