@@ -1128,7 +1128,7 @@ __global__ __launch_bounds__(kWideThreads) void wide_law_kernel(const float* __r
     }
     double S = 0.0;
     for (int c = 0; c < n_chunks; ++c)
-      if (pp[c].m > -INFINITY) S += pp[c].s * exp(pp[c].m - M);
+      if (pp[c].m > -INFINITY) S = fma(pp[c].s, exp(pp[c].m - M), S);   // (wide_hist adds the same way)
     s_M = M;
     s_S = S;
     s_nf = nf || !(isfinite(S) && S > 0.0);
@@ -1263,8 +1263,8 @@ __global__ __launch_bounds__(kWideThreads) void wide_law_kernel(const float* __r
 // The same law over many workgroups, for rows of more than two chunks. One
 // workgroup per row leaves most of the chip idle (28 rows on 256 CUs) and walks
 // a row in 149 rounds of block scans: 557 us for 28 rows of 151936. Here, with
-// the same ids and probabilities bit for bit, 24 + 15 + 14 + 34 us (four
-// requests' accept step of depth 3: 597 -> 124 us):
+// the same ids and probabilities bit for bit, 26 + 15 + 10 + 12 us (the accept
+// step of four requests of depth 3: 597-612 -> 121-138 us):
 //  1. wide_hist: per chunk, the count and fixed-point mass of each bin of the
 //     distance from the row's maximum (bins are monotone in the logit; integer
 //     sums, so the order of the additions does not matter);
@@ -1325,7 +1325,7 @@ __global__ __launch_bounds__(kSampThreads) void wide_hist(const float* __restric
   const WideRow wr = wide_row(hist, n_chunks, row);
   __shared__ unsigned long long s_mass[kWideBins];
   __shared__ uint32_t s_cnt[kWideBins];
-  __shared__ double s_wm[NWV], s_term[kSampThreads];
+  __shared__ double s_wm[NWV], s_sum[kSampThreads], s_exp[kSampThreads];
   __shared__ int s_wnf[NWV];
   __shared__ uint64_t s_wk[NWV];
   __shared__ double s_S;
@@ -1340,7 +1340,8 @@ __global__ __launch_bounds__(kSampThreads) void wide_hist(const float* __restric
     const int id = chunk * kChunk + e * kSampThreads + tid;
     v[e] = id < V ? lr[id] : 0.f;
   }
-  // fp64 max / sum-exp combine in fixed chunk order (as build_law).
+  // fp64 max / sum-exp combine in fixed chunk order, each chunk's product and
+  // its addition rounded once (as wide_law_kernel: the same S to the last bit).
   double M = -INFINITY;
   int nf = 0;
   uint64_t best = 0ull;
@@ -1367,11 +1368,13 @@ __global__ __launch_bounds__(kSampThreads) void wide_hist(const float* __restric
   double S = 0.0;
   for (int c0 = 0; c0 < n_chunks; c0 += kSampThreads) {
     const int c = c0 + tid;
-    s_term[tid] = (c < n_chunks && pp[c].m > -INFINITY) ? pp[c].s * exp(pp[c].m - M) : 0.0;
+    const bool some = c < n_chunks && pp[c].m > -INFINITY;
+    s_sum[tid] = some ? pp[c].s : 0.0;
+    s_exp[tid] = some ? exp(pp[c].m - M) : 0.0;
     __syncthreads();
     if (tid == 0) {
       const int n = n_chunks - c0 < kSampThreads ? n_chunks - c0 : kSampThreads;
-      for (int i = 0; i < n; ++i) S += s_term[i];
+      for (int i = 0; i < n; ++i) S = fma(s_sum[i], s_exp[i], S);
     }
     __syncthreads();
   }

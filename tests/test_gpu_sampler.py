@@ -161,6 +161,21 @@ def test_wide_law_over_many_workgroups(gpu, V, cfg):
         assert int(smp[r]) == S.choice(want, u[r]), r
 
 
+@pytest.mark.parametrize("cfg", [S.SamplerConfig(0.6, 0.95, 0), S.SamplerConfig(1.0, 1.0, 0),
+                                 S.SamplerConfig(0.8, 0.9, 200)])
+def test_wide_laws_agree_bit_for_bit(gpu, cfg):
+    """Two chunks of ids take one workgroup per row, three take the binned
+    launches: one masked id past the second chunk changes the launches and
+    nothing else, so ids, probabilities and draws are the same bits."""
+    rng = np.random.default_rng(11)
+    a = rng.normal(0, 3, (48, 8192)).astype(np.float32)
+    b = np.concatenate([a, np.full((48, 1), -np.inf, np.float32)], axis=1)
+    u = rng.random(48)
+    one, many = (_sample_rows(t, cfg, u, ld=_bound(cfg, 8193)) for t in (a, b))
+    for x, y in zip(one, many):
+        assert np.array_equal(x, y)
+
+
 def test_output_rows_use_the_given_stride(gpu):
     """Greedy with top_k = 20 (support 1) written at a row stride of 20: every
     row's slot 0 is its argmax and the rest is padded (-1, 0)."""
