@@ -430,12 +430,11 @@ MTP_API int mtp_gather_qmv_affine4(const void* x, const void* x2, const uint32_t
     p.active = active;
     p.w_estride = (long long)rows_per_expert * (K / 2);
     p.s_estride = (long long)rows_per_expert * (K / group_size);
-    p.M = max_rows_per_expert;
     p.N = N;
     p.K = K;
     p.ldx = K;
     p.ldy = N;
-    inplace_launch(p, 4, group_size, max_rows_per_expert, emode == E_DUAL_SWIGLU, (hipStream_t)stream);
+    inplace_launch(p, 4, group_size, emode == E_DUAL_SWIGLU, (hipStream_t)stream);
     return launch_check(who);
   }
   QmmParams p = base_params(x, w0, s0, b0, y, 32, N, K, group_size);

@@ -73,7 +73,7 @@ static int qmv_affine_run(const void* x, const float* xsums, const void* w, cons
   p.K = K;
   p.ldx = K;
   p.ldy = N;
-  inplace_launch(p, bits, group_size, M, false, (hipStream_t)stream);
+  inplace_launch(p, bits, group_size, false, (hipStream_t)stream);
   return launch_check(who);
 }
 

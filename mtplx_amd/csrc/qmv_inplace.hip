@@ -2,26 +2,17 @@
 // a format and a row count, for one matrix or for the experts of a sort.
 #include "qmv_inplace.hpp"
 
-#include <climits>
+#include <limits.h>
 
 namespace mtp {
 
-template <int BITS, int GS, int R, bool DUAL, bool VEC, bool XS, int NW, int KS, int ND>
-static void inplace_run(InplaceParams p, hipStream_t st) {
-  using S = InplaceShape<BITS, GS, R, DUAL, NW, KS, ND>;
-  auto k = qmv_inplace_kernel<BITS, GS, R, DUAL, VEC, XS, NW, KS, ND>;
-  constexpr int lds = (int)S::lds();
-  // Workgroups per CU by LDS, at most two.
-  constexpr int per_cu = 160 * 1024 / (lds + S::FIXED) >= 2 ? 2 : 1;
-  static_assert(lds + S::FIXED <= 160 * 1024, "a workgroup's LDS");
+// Launches kernel k, of ``threads`` threads and ``lds`` bytes of LDS: a
+// workgroup per item, at most as many as the CUs hold (two each at most).
+template <class Kernel>
+static void inplace_run(Kernel k, const InplaceParams& p, int threads, int lds, long long items, hipStream_t st) {
   (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  p.ntile = cdiv(p.N, S::OC);
-  int grid = per_cu * device_cus();
-  if (!p.active) {
-    const long long items = (long long)p.ntile * cdiv(p.M, R);
-    if (items < grid) grid = (int)items;
-  }
-  hipLaunchKernelGGL(k, dim3(grid), dim3(NW * 64), lds, st, p);
+  const long long most = (160 * 1024 / lds >= 2 ? 2ll : 1ll) * device_cus();
+  hipLaunchKernelGGL(k, dim3((unsigned)(items < most ? items : most)), dim3(threads), lds, st, p);
 }
 
 // One matrix: 32 columns a workgroup, K split over all of its waves, in the
@@ -30,41 +21,41 @@ static void inplace_run(InplaceParams p, hipStream_t st) {
 // 23.9; two workgroups of 4 waves 23.8 and 27.1, with one stage 25.8 and
 // 33.3); more rows, 4 waves, whose stages hold 16 rows of x (32768 x 5120, 16
 // rows: 40.5 us, with one stage 48.8).
-template <int BITS, int GS, bool VEC, bool XS>
-static void inplace_dense(const InplaceParams& p, int max_rows, hipStream_t st) {
-  if (max_rows <= 4)
-    inplace_run<BITS, GS, 4, false, VEC, XS, 8, 8, 2>(p, st);
-  else
-    inplace_run<BITS, GS, 16, false, VEC, XS, 4, 4, 2>(p, st);
+template <int BITS, int GS, int R, bool VEC, bool XS, int NW>
+static void inplace_dense(InplaceParams p, hipStream_t st) {
+  using S = InplaceShape<BITS, GS, R, false, NW, NW, 2>;
+  static_assert(S::lds() <= 160 * 1024, "a workgroup's LDS");
+  p.ntile = cdiv(p.N, S::OC);
+  inplace_run(qmv_inplace_kernel<BITS, GS, R, VEC, XS, NW>, p, NW * 64, (int)S::lds(),
+              (long long)p.ntile * cdiv(p.M, R), st);
+}
+
+template <int GS, bool DUAL, bool VEC>
+static void inplace_experts(InplaceParams p, hipStream_t st) {
+  using E = InplaceExperts<GS, DUAL, VEC>;
+  static_assert(2 * E::lds() <= 160 * 1024, "two workgroups per CU");
+  p.ntile = cdiv(p.N, E::Few::OC);
+  inplace_run(qmv_inplace_experts<GS, DUAL, VEC>, p, 256, (int)E::lds(), LLONG_MAX, st);   // (the device knows how many items)
 }
 
 template <int BITS, int GS, bool DUAL, bool VEC>
-static void inplace_rows(InplaceParams p, int max_rows, hipStream_t st) {
-  if constexpr (!DUAL) {
-    if (!p.active) {
-      if constexpr (BITS == 4 && GS <= 64) {
-        if (p.xsums) return inplace_dense<BITS, GS, VEC, true>(p, max_rows, st);   // the cross-row lane
-      }
-      return inplace_dense<BITS, GS, VEC, false>(p, max_rows, st);
-    }
-  }
-  // Experts: those with at most 4 rows, then the others in tiles of 16. Two
-  // K parts and two column groups (the pair: its matrices) per workgroup: an
-  // item is twice as long as with four parts, and K = 1536 has 6 chunks (down
-  // 48 us against 59, gate|up 90 against 92).
+static void inplace_rows(const InplaceParams& p, hipStream_t st) {
   if constexpr (BITS == 4 && GS >= 64) {
-    p.m_lo = 1;
-    p.m_hi = 4;
-    inplace_run<BITS, GS, 4, DUAL, VEC, false, 4, 2, 1>(p, st);
-    if (max_rows <= 4) return;
-    p.m_lo = 5;
-    p.m_hi = INT_MAX;
-    inplace_run<BITS, GS, 16, DUAL, VEC, false, 4, 2, 1>(p, st);
+    if (p.active) return inplace_experts<GS, DUAL, VEC>(p, st);
+  }
+  if constexpr (!DUAL) {
+    if constexpr (BITS == 4 && GS <= 64) {
+      if (p.xsums)   // the cross-row lane
+        return p.M <= 4 ? inplace_dense<BITS, GS, 4, VEC, true, 8>(p, st)
+                        : inplace_dense<BITS, GS, 16, VEC, true, 4>(p, st);
+    }
+    return p.M <= 4 ? inplace_dense<BITS, GS, 4, VEC, false, 8>(p, st)
+                    : inplace_dense<BITS, GS, 16, VEC, false, 4>(p, st);
   }
 }
 
 template <int BITS, int GS, bool DUAL>
-static void inplace_vec(const InplaceParams& p, int max_rows, hipStream_t st) {
+static void inplace_vec(const InplaceParams& p, hipStream_t st) {
   // Scales straight to LDS in 16-byte pieces of eight groups where rows hold
   // whole pieces and the arrays are so aligned; else element by element. x may
   // start at any element too.
@@ -72,26 +63,26 @@ static void inplace_vec(const InplaceParams& p, int max_rows, hipStream_t st) {
   const bool vec = (p.K / GS) % 8 == 0 && aligned(p.x) && aligned(p.s0) && aligned(p.b0) &&
                    (!DUAL || (aligned(p.s1) && aligned(p.b1)));
   if (vec) {
-    inplace_rows<BITS, GS, DUAL, true>(p, max_rows, st);
+    inplace_rows<BITS, GS, DUAL, true>(p, st);
   } else {
-    inplace_rows<BITS, GS, DUAL, false>(p, max_rows, st);
+    inplace_rows<BITS, GS, DUAL, false>(p, st);
   }
 }
 
-void inplace_launch(const InplaceParams& p, int bits, int gs, int max_rows, bool dual, hipStream_t st) {
+void inplace_launch(const InplaceParams& p, int bits, int gs, bool dual, hipStream_t st) {
   if (dual) {   // 4-bit, groups 64/128, K % 256 == 0, aligned scales (checked by the caller)
     if (gs == 64)
-      inplace_vec<4, 64, true>(p, max_rows, st);
+      inplace_vec<4, 64, true>(p, st);
     else
-      inplace_vec<4, 128, true>(p, max_rows, st);
+      inplace_vec<4, 128, true>(p, st);
   } else if (bits == 4) {
-    if (gs == 32) inplace_vec<4, 32, false>(p, max_rows, st);
-    else if (gs == 64) inplace_vec<4, 64, false>(p, max_rows, st);
-    else inplace_vec<4, 128, false>(p, max_rows, st);
+    if (gs == 32) inplace_vec<4, 32, false>(p, st);
+    else if (gs == 64) inplace_vec<4, 64, false>(p, st);
+    else inplace_vec<4, 128, false>(p, st);
   } else {
-    if (gs == 32) inplace_vec<8, 32, false>(p, max_rows, st);
-    else if (gs == 64) inplace_vec<8, 64, false>(p, max_rows, st);
-    else inplace_vec<8, 128, false>(p, max_rows, st);
+    if (gs == 32) inplace_vec<8, 32, false>(p, st);
+    else if (gs == 64) inplace_vec<8, 64, false>(p, st);
+    else inplace_vec<8, 128, false>(p, st);
   }
 }
 

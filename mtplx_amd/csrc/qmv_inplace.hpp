@@ -52,6 +52,8 @@
 
 #include "qmv_common.hpp"
 
+#include <limits.h>
+
 namespace mtp {
 
 struct InplaceParams {
@@ -72,7 +74,6 @@ struct InplaceParams {
   long long s_estride;     // scales between experts
   int M, N, K, ldx, ldy;
   int ntile;               // column tiles
-  int m_lo, m_hi;          // experts with m_lo <= rows <= m_hi
 };
 
 constexpr int kInList = 128;    // experts listed in LDS at a time
@@ -106,9 +107,16 @@ struct InplaceShape {
   static constexpr int OC = DUAL ? TC / 2 : TC;       // output columns per tile
   static constexpr int SCAL = 2 * TC * SROW;       // one segment: scales [TC][row], then biases
   static constexpr int RED = 2 * NW * XR * COLS * 4;
-  static constexpr size_t lds() { return (size_t)NW * D * STAGE + RED + 2 * SCAL; }
+  // What comes first in LDS: the experts listed, and the items described.
+  struct Lists {
+    int4 item[ITEMS];                // expert, column tile, first row, rows
+    int rows[ITEMS][XR];             // x row of each staged row
+    int e[kInList], r0[kInList], cum[kInList + 1];   // expert, its first row, row tiles before it
+    int wcnt[NW], wtil[NW];          // per wave of the scan
+  };
+  static constexpr int LISTS = (sizeof(Lists) + 255) & ~255;
+  static constexpr size_t lds() { return (size_t)LISTS + NW * D * STAGE + RED + 2 * SCAL; }
   static_assert(GRP % GPC == 0 && GRP % 8 == 0, "segments of whole chunks and 16-byte pieces");
-  static constexpr int FIXED = 2 * kInList * 4 + (kInList + 1) * 4 + 8 * NW + ITEMS * (16 + 4 * XR) + 64;   // static LDS
   static_assert((GRP / 8) % 2 == 1, "odd rows");
   static_assert(XI >= 1, "a chunk of x is at least one load");
 };
@@ -132,11 +140,15 @@ __device__ __forceinline__ void group_vals(const unsigned char* at, float (&o)[G
   for (int u = 0; u < GPC; ++u) o[u] = __uint_as_float((u & 1) ? (v[u >> 1] & 0xffff0000u) : (v[u >> 1] << 16));
 }
 
+// The work of one workgroup, number ``bid`` of the grid: all rows, or the rows
+// of the experts with m_lo <= rows <= m_hi. Returns (to every thread) whether
+// an expert has more rows than m_hi.
 // VEC: scales straight to LDS, and x 16-byte aligned (else scales element by
 // element, and x too where it is not aligned). XS: the bias term
 // takes its group sums from the caller's chunk-sum table (p.xsums).
 template <int BITS, int GS, int R, bool DUAL, bool VEC, bool XS, int NW, int KS, int ND>
-__global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inplace_kernel(InplaceParams p) {
+__device__ __forceinline__ bool inplace_body(const InplaceParams& p, unsigned char* const lds_base, int bid, int m_lo,
+                                             int m_hi) {
   using S = InplaceShape<BITS, GS, R, DUAL, NW, KS, ND>;
   constexpr int COLS = S::COLS;
   static_assert(!DUAL || NW == 2 * KS, "the pair: half the waves on each matrix");
@@ -146,11 +158,8 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
   constexpr int SPG = GS / 32;          // MFMA steps per group
   constexpr int LPR = S::XB / 16;       // lanes per x row in a load
   constexpr int NL = S::WI + S::XI;     // loads per stage
-  extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int s_e[kInList], s_r0[kInList], s_cum[kInList + 1];
-  __shared__ int s_wcnt[NW], s_wtil[NW];
-  __shared__ int4 s_item[S::ITEMS];          // expert, column tile, first row, rows
-  __shared__ int s_rows[S::ITEMS][S::XR];    // x row of each staged row
+  auto& L = *reinterpret_cast<typename S::Lists*>(lds_base);
+  unsigned char* const smem = lds_base + S::LISTS;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -210,6 +219,7 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
 
   // Base of experts [l0, l0 + kInList) of the active list, then their items.
   const int n_active = p.active ? p.active[0] : 1;
+  int more = 0;   // an expert above m_hi
   for (int l0 = 0; l0 < n_active; l0 += kInList) {
     int n_list = 1;
     __syncthreads();
@@ -226,7 +236,8 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
           r0 = p.expert_off[e];
           rows = p.expert_off[e + 1] - r0;
         }
-        const bool in = t < l1 && rows >= p.m_lo && rows <= p.m_hi;
+        const bool in = t < l1 && rows >= m_lo && rows <= m_hi;
+        const int above = __any(t < l1 && rows > m_hi) ? 1 << 16 : 0;
         const int tiles = in ? (rows + S::XR - 1) / S::XR : 0;
         const unsigned long long bal = __ballot(in);
         int inc = tiles;
@@ -236,40 +247,42 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
           if (lane >= off) inc += v;
         }
         if (lane == 63) {
-          s_wcnt[wave] = __popcll(bal);
-          s_wtil[wave] = inc;
+          L.wcnt[wave] = __popcll(bal) + above;
+          L.wtil[wave] = inc;
         }
         __syncthreads();
         int at = nl, before = nt;
         for (int w = 0; w < NW; ++w) {
+          const int c = L.wcnt[w] & 0xffff;
           if (w < wave) {
-            at += s_wcnt[w];
-            before += s_wtil[w];
+            at += c;
+            before += L.wtil[w];
           }
-          nl += s_wcnt[w];
-          nt += s_wtil[w];
+          nl += c;
+          nt += L.wtil[w];
+          more |= L.wcnt[w] >> 16;
         }
         if (in) {
           const int i = at + __popcll(bal & ((1ull << lane) - 1ull));
-          s_e[i] = e;
-          s_r0[i] = r0;
-          s_cum[i] = before + inc - tiles;
+          L.e[i] = e;
+          L.r0[i] = r0;
+          L.cum[i] = before + inc - tiles;
         }
         __syncthreads();
       }
       n_list = nl;
-      if (tid == 0) s_cum[nl] = nt;
+      if (tid == 0) L.cum[nl] = nt;
     } else if (tid == 0) {
-      s_e[0] = 0;
-      s_r0[0] = 0;
-      s_cum[0] = 0;
-      s_cum[1] = (p.M + S::XR - 1) / S::XR;
+      L.e[0] = 0;
+      L.r0[0] = 0;
+      L.cum[0] = 0;
+      L.cum[1] = (p.M + S::XR - 1) / S::XR;
     }
     __syncthreads();
-    const int n_items = s_cum[n_list] * p.ntile;
+    const int n_items = L.cum[n_list] * p.ntile;
 
-    // This workgroup's items blockIdx.x, + gridDim.x, ..., S::ITEMS at a time.
-    for (int i0 = blockIdx.x; i0 < n_items; i0 += S::ITEMS * gridDim.x) {
+    // This workgroup's items bid, + gridDim.x, ..., S::ITEMS at a time.
+    for (int i0 = bid; i0 < n_items; i0 += S::ITEMS * gridDim.x) {
       const int left = (n_items - i0 + (int)gridDim.x - 1) / (int)gridDim.x;
       const int ni = left < S::ITEMS ? left : S::ITEMS;
       __syncthreads();   // the last items' readers are done
@@ -280,15 +293,15 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
         int lo = 0, hi = n_list;      // its expert: the last with cum <= rt
         while (hi - lo > 1) {
           const int mid = (lo + hi) >> 1;
-          if (s_cum[mid] <= rt) lo = mid; else hi = mid;
+          if (L.cum[mid] <= rt) lo = mid; else hi = mid;
         }
-        const int e = s_e[lo];
-        const int rows = p.active ? p.expert_off[e + 1] - s_r0[lo] : p.M;
-        const int t0 = (rt - s_cum[lo]) * S::XR;
+        const int e = L.e[lo];
+        const int rows = p.active ? p.expert_off[e + 1] - L.r0[lo] : p.M;
+        const int t0 = (rt - L.cum[lo]) * S::XR;
         const int n = rows - t0 < S::XR ? rows - t0 : S::XR;
-        const int row = s_r0[lo] + t0 + (r < n ? r : n - 1);
-        if (r == 0) s_item[it] = make_int4(e, w - rt * p.ntile, s_r0[lo] + t0, n);
-        s_rows[it][r] = p.rowmap ? (int)p.rowmap[row] : row;
+        const int row = L.r0[lo] + t0 + (r < n ? r : n - 1);
+        if (r == 0) L.item[it] = make_int4(e, w - rt * p.ntile, L.r0[lo] + t0, n);
+        L.rows[it][r] = p.rowmap ? (int)p.rowmap[row] : row;
       }
       __syncthreads();
 
@@ -299,8 +312,8 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
       uint32_t w_off[S::WI];
       const uint16_t* x_ptr[S::XI];
       auto set_item = [&](int it) {
-        const int e = __builtin_amdgcn_readfirstlane(s_item[it].x);
-        const int tile = __builtin_amdgcn_readfirstlane(s_item[it].y);
+        const int e = __builtin_amdgcn_readfirstlane(L.item[it].x);
+        const int tile = __builtin_amdgcn_readfirstlane(L.item[it].y);
         const int n0 = tile * S::OC + (DUAL ? 0 : cg * COLS);
         w_base = (DUAL && cg ? p.w1 : p.w0) + e * p.w_estride;
 #pragma unroll
@@ -312,14 +325,14 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
 #pragma unroll
         for (int i = 0; i < S::XI; ++i) {
           const int r = i * (64 / LPR) + x_r;
-          x_ptr[i] = p.x + (size_t)s_rows[it][r] * p.ldx;
+          x_ptr[i] = p.x + (size_t)L.rows[it][r] * p.ldx;
         }
       };
       // The scales and biases of segment sg of item it, into buffer (it * nseg
       // + sg) % 2, by the whole workgroup: 16-byte pieces straight to LDS (VEC;
       // a row's pieces past its last repeat it), else element by element.
       auto load_scales = [&](int it, int sg) {
-        const int4 im = s_item[it];
+        const int4 im = L.item[it];
         const int n0 = im.y * S::OC;
         const int g0 = sg * S::GRP;
         const int ng = sgroups - g0 < S::GRP ? sgroups - g0 : S::GRP;
@@ -553,7 +566,7 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
             for (int h = 0; h < S::PW; ++h) acc[h][ct][i] = 0.f;
           }
         lds_barrier();
-        const int4 im = s_item[it];
+        const int4 im = L.item[it];
         for (int idx = tid; idx < S::XR * S::OC; idx += NT) {
           const int m = idx / S::OC, c = idx - m * S::OC;
           const int col = im.y * S::OC + c;
@@ -632,11 +645,41 @@ __global__ __launch_bounds__(NW * 64, R == 16 && ND == 1 ? 2 : 1) void qmv_inpla
       wait_vm<0>();   // the stages are loaded again for the next items
     }
   }
+  return more != 0;
 }
 
-// Launches it for bits 4/8 and groups 32/64/128; ``max_rows``: M, or the most
-// rows an expert can have. ``dual``: the fused SwiGLU pair (4-bit, groups
-// 64/128, K % 256 == 0).
-void inplace_launch(const InplaceParams& p, int bits, int gs, int max_rows, bool dual, hipStream_t st);
+// One matrix.
+template <int BITS, int GS, int R, bool VEC, bool XS, int NW>
+__global__ __launch_bounds__(NW * 64, 1) void qmv_inplace_kernel(InplaceParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  inplace_body<BITS, GS, R, false, VEC, XS, NW, NW, 2>(p, smem, blockIdx.x, 1, INT_MAX);
+}
+
+// Experts: those with at most 4 rows in tiles of 4, then, where there are such,
+// the others in tiles of 16, all in one launch. A launch for each class costs
+// the small calls, which wait for launches (4 rows x 8 of 256 experts through
+// the three gathers of an unsorted block: 270-281 us, 258 with one launch each;
+// 16 rows x 8 through the sorted block: 188 and 177; 512 rows x 8: 1045 and
+// 1023). The second class is handed out from the last workgroup on: the first
+// ones may hold an item more of the first. Two K parts and two column groups
+// (the pair: its matrices) per workgroup: an item is twice as long as with four
+// parts, and K = 1536 has 6 chunks (down 48 us against 59, gate|up 90 against 92).
+template <int GS, bool DUAL, bool VEC>
+struct InplaceExperts {
+  using Few = InplaceShape<4, GS, 4, DUAL, 4, 2, 1>;
+  using Many = InplaceShape<4, GS, 16, DUAL, 4, 2, 1>;
+  static constexpr size_t lds() { return Few::lds() > Many::lds() ? Few::lds() : Many::lds(); }
+  static_assert(Few::OC == Many::OC, "one column tile for both classes");
+};
+template <int GS, bool DUAL, bool VEC>
+__global__ __launch_bounds__(256, 2) void qmv_inplace_experts(InplaceParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (inplace_body<4, GS, 4, DUAL, VEC, false, 4, 2, 1>(p, smem, blockIdx.x, 1, 4))
+    inplace_body<4, GS, 16, DUAL, VEC, false, 4, 2, 1>(p, smem, gridDim.x - 1 - blockIdx.x, 5, INT_MAX);
+}
+
+// Launches it for bits 4/8 and groups 32/64/128 (experts: 4 bits, groups 64/128).
+// ``dual``: the experts' fused SwiGLU pair (K % 256 == 0).
+void inplace_launch(const InplaceParams& p, int bits, int gs, bool dual, hipStream_t st);
 
 }  // namespace mtp

@@ -118,3 +118,54 @@ def test_experts(gpu, E, T, k, H, F, gs, skew):
     gb, ub = round_to_bf16(gate), round_to_bf16(up)
     want = round_to_bf16(round_to_bf16(gb / (1.0 + np.exp(-gb))) * ub)
     assert_swiglu_close(bf16_values(h), gb, ub, want, what="SwiGLU pair")
+
+
+def _gather_nodes(call):
+    """Kernels that ``call`` launches: the nodes of its captured graph."""
+    import ctypes
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        call()
+    n = ctypes.c_size_t()
+    hip = ctypes.CDLL(None)   # torch's HIP runtime is mapped
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("emode", [0, 3])
+def test_both_row_classes_in_one_launch(gpu, emode):
+    """A gather whose experts have 1..4 rows and more is one kernel (small
+    routed calls wait for launches), and a row's output has the same bits
+    whichever class its expert falls in."""
+    from mtplx_amd import _lib
+    from mtplx_amd.moe_sorted_gather import expert_sort
+    rng = np.random.default_rng(8)
+    E, K, F = 5, 2048, 160
+    gate, up = (tuple(a.reshape(E, F, -1) for a in make_affine4_weights(rng, E * F, K, 64)) for _ in range(2))
+    gd, ud = ((u32(t[0]), from_bits(t[1]), from_bits(t[2])) for t in (gate, up))
+    x = randn_bf16(rng, (24, K))
+
+    def gather(ids):
+        es = expert_sort(torch.from_numpy(ids).reshape(-1, 1).cuda(), E)
+        y = torch.zeros((ids.size, F), dtype=torch.bfloat16, device="cuda")
+        args = (x.data_ptr(), None, es.row_map.data_ptr(), es.expert_off.data_ptr(), es.active.data_ptr(),
+                *(t.data_ptr() for t in gd), *(t.data_ptr() if emode else None for t in ud), y.data_ptr(), ids.size, E, F,
+                K, 64, 0, emode, F, None, 0)
+        run = lambda: _lib.call("mtp_gather_qmv_affine4", *args,   # noqa: E731
+                                torch.cuda.current_stream().cuda_stream)
+        return es, y, run
+
+    ids = np.array([1] * 3 + [4] * 17 + [0] * 4, dtype=np.int32)   # both classes, two row tiles
+    es, y, run = gather(ids)
+    run()
+    torch.cuda.synchronize()
+    assert not torch.isnan(y.float()).any()
+    flat = y[es.inv_order.long()].clone()
+    es1, y1, run1 = gather(np.array([4], dtype=np.int32).repeat(3))   # x rows 0..2 of expert 4, in the small class
+    es2, y2, run2 = gather(np.array([4], dtype=np.int32).repeat(20))  # and in the large one
+    run1()
+    run2()
+    torch.cuda.synchronize()
+    assert torch.equal(y1.view(torch.int16), y2[:3].view(torch.int16))
+    assert torch.equal(y2[3:20].view(torch.int16), flat[3:20].view(torch.int16))
+    assert _gather_nodes(run) == 1
