@@ -208,11 +208,15 @@ class _Workspaces:
     """One zero-initialised byte buffer per (device, stream, tag), grown on demand.
 
     Kernels keep self-resetting arrival counters in their workspace, so a
-    buffer is zero-filled only when it is (re)allocated.
+    buffer is zero-filled only when it is (re)allocated. A captured graph
+    replays with the address it was recorded with, so an outgrown buffer stays
+    allocated (sizes at least double: those kept are together no larger than
+    the one in use).
     """
 
     def __init__(self):
         self._bufs: dict = {}
+        self._outgrown: list = []
 
     def get(self, nbytes: int, tag: str, device=None):
         import torch
@@ -225,6 +229,7 @@ class _Workspaces:
             size = max(int(nbytes), 256)
             if buf is not None:
                 size = max(size, 2 * buf.numel())
+                self._outgrown.append(buf)
             buf = torch.zeros(size, dtype=torch.uint8, device=dev)
             self._bufs[key] = buf
         return buf

@@ -220,3 +220,33 @@ def test_tiles_match_oracle(gpu, m, n, k, gs):
     # a workspace one byte short is refused
     with pytest.raises(_lib.MtpError):
         _lib.call("mtp_qmm_affine4_tiles", x.data_ptr(), *args[:-2], ws.numel() - 1, args[-1])
+
+
+def test_captured_call_outlives_a_larger_one(gpu):
+    """A prompt-chunk matmul captured on a stream replays right after a larger
+    call on that stream has outgrown its workspace and other tensors were
+    allocated (the captured address must still be the call's own)."""
+    from mtplx_amd.verify_kernels import quantized_matmul
+    from oracle.qmv import make_affine4_weights
+    from tests.gpu_util import from_bits, randn_bf16, u32
+    rng = np.random.default_rng(13)
+    n, k = 256, 4096
+    triple = tuple(f(a) for f, a in zip((u32, from_bits, from_bits), make_affine4_weights(rng, n, k, 64)))
+    x, large = randn_bf16(rng, (100, k)), randn_bf16(rng, (700, k))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        want = quantized_matmul(x, *triple)   # the stream's workspace, sized for 100 rows
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        got = quantized_matmul(x, *triple)
+    with torch.cuda.stream(s):
+        for _ in range(3):
+            quantized_matmul(large, *triple)
+            junk = [torch.full((1 << 20,), 255, dtype=torch.uint8, device="cuda") for _ in range(8)]
+            got.zero_()
+            g.replay()
+            s.synchronize()
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+            assert all(bool((j == 255).all()) for j in junk)   # and the replay wrote into nobody else's memory
