@@ -188,6 +188,7 @@ __global__ __launch_bounds__(kTiThreads, 2) void qmm_tiles_kernel(TilesParams p)
   // slot (5 loads) may be in flight; past the barrier every wave's x of quad q is in
   // LDS, and nobody reads the other buffer any more.
   auto step = [&](TileQuad& cur, int q) {
+    asm volatile("" ::: "memory");   // (no load moves past the wait, which counts them)
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(5));
     lds_barrier();
     stage(q + 1);
@@ -195,12 +196,18 @@ __global__ __launch_bounds__(kTiThreads, 2) void qmm_tiles_kernel(TilesParams p)
     asm volatile("" ::: "memory");
     load_quad(cur, q + 2);
   };
+  // An odd last quad leaves the loop in its middle: with a path through the loop
+  // that skips ring1, ring0's loads may be the newest that the compiler knows
+  // of, and it waits for everything in flight (vmcnt(0), the DMAs just issued
+  // among it) before it reads ring0.
   int q = 0;
-  do {
+  while (true) {
     step(ring0, q);
-    if (q + 1 < Q) step(ring1, q + 1);
+    if (q + 1 >= Q) break;
+    step(ring1, q + 1);
     q += 2;
-  } while (q < Q);
+    if (q >= Q) break;
+  }
 
   const int col = 32 * ct + c32;
   if (!has_tile || col >= p.N) return;
