@@ -188,6 +188,7 @@ def test_one_workspace_serves_shapes_in_turn(gpu):
     (130, 5120, 512, 64),     # 120 workgroups of two quads
     (193, 8224, 768, 128),    # more workgroups than CUs: no K parts
     (65, 4096, 12288, 64),    # 48 quads
+    (449, 4128, 12544, 64),   # 264 workgroups (more than CUs, fewer than two each) of 49 quads: 3 uneven K parts
 ])
 def test_tiles_match_oracle(gpu, m, n, k, gs):
     """mtp_qmm_affine4_tiles at the edges of its row tiles (64), column groups
@@ -220,6 +221,24 @@ def test_tiles_match_oracle(gpu, m, n, k, gs):
     # a workspace one byte short is refused
     with pytest.raises(_lib.MtpError):
         _lib.call("mtp_qmm_affine4_tiles", x.data_ptr(), *args[:-2], ws.numel() - 1, args[-1])
+
+
+def test_tiles_past_one_launch(gpu):
+    """More rows than one launch of the tiles kernel takes (8192), in two
+    launches that share a workspace: against the oracle, and the second
+    launch's rows as alone."""
+    from mtplx_amd.verify_kernels import TILES_ROWS, quantized_matmul
+    from oracle.qmv import make_affine4_weights
+    from tests.gpu_util import from_bits, randn_bf16, u32
+    rng = np.random.default_rng(12)
+    m, n, k = TILES_ROWS + 65, 40, 512
+    w, s, bb = make_affine4_weights(rng, n, k, 64)
+    x, triple = randn_bf16(rng, (m, k)), (u32(w), from_bits(s), from_bits(bb))
+    y = quantized_matmul(x, *triple)
+    tail = quantized_matmul(x[TILES_ROWS:], *triple)
+    torch.cuda.synchronize()
+    assert_close(bf16_values(y), round_to_bf16(qmm_affine4(bits(x), w, s, bb, 64)), what="two launches")
+    assert torch.equal(y[TILES_ROWS:].view(torch.int16), tail.view(torch.int16))
 
 
 def test_captured_call_outlives_a_larger_one(gpu):
