@@ -239,14 +239,28 @@ using namespace mtp;
 
 // K parts. A grid of fewer workgroups than CUs is split over them (128 rows,
 // 5120 x 17408, 80 workgroups: 94.5 us whole, 44.4 in 3 parts; 65 rows, 1024 x
-// 5120, 16 workgroups: 32.7, in 8 parts 16.0), two quads a part at least; one of
-// less than two per CU only where a part is long (512 rows, 5120 x 17408, 320
-// workgroups: 143.8 us, in 3 parts 125.0; 5120 x 5120: 49.5 and 51.1).
+// 5120, 16 workgroups: 32.7, in 8 parts 16.0), two quads a part at least. One of
+// one to two per CU takes the split with the least estimated time: a CU of the
+// fullest XCD runs ceil(w s / CUs) parts of Q / s quads, 1.1 us each, and the
+// parts cost a launch and a pass over their sums, 5 us and 8 bytes a sum at 5
+// TB/s. Measured for one, two and three parts (K 1536 to 17408 of nine grids),
+// it takes one within 2% of the best:
+// 35 workgroups on an XCD's 32 CUs (448 rows, 5120 x 17408: 137, 125, 114 us; K
+// 5120: 47.2, 48.1, 46.6), 40 (512 rows: 143, 129, 120; K 7168 62.8, 61.0, 59.3;
+// K 5120 47.8, 48.7, 48.2), 48 (768 rows, 4096 x 17408: 150, 136, 146; K 7168
+// 64.9, 65.1, 71.8), 60 (768 rows, 5120 x 17408: 160, 169, 174).
 static int tiles_split(int M, int N, int K) {
   const long long blocks = (long long)cdiv(M, kTiRows) * cdiv(cdiv(N, 32), 4);
   const int cus = device_cus(), Q = K / 256;
   if (blocks >= 2 * cus) return 1;
-  if (blocks >= cus) return Q >= 48 ? 3 : 1;
+  if (blocks >= cus) {
+    const int w = cdiv(M, kTiRows) * cdiv(cdiv(cdiv(N, 32), 4), 8);   // workgroups on the fullest XCD
+    auto us = [&](int s) {
+      return 1.1 * Q * cdiv(8 * w * s, cus) / s + (s > 1 ? 5.0 + s * ((double)M * N) * 8.0 / 5e6 : 0.0);
+    };
+    const int s = us(2) < us(1) ? 2 : 1;
+    return us(3) < us(s) ? 3 : s;   // (at most Q: below 3 quads the parts cost more than they can save)
+  }
   long long s = cus / blocks;
   if (s > 8) s = 8;
   if (s > Q / 2) s = Q / 2;

@@ -189,6 +189,7 @@ def test_one_workspace_serves_shapes_in_turn(gpu):
     (193, 8224, 768, 128),    # more workgroups than CUs: no K parts
     (65, 4096, 12288, 64),    # 48 quads
     (449, 4128, 12544, 64),   # 264 workgroups (more than CUs, fewer than two each) of 49 quads: 3 uneven K parts
+    (705, 4000, 9472, 64),    # 384 of 37 quads: 2 uneven K parts
 ])
 def test_tiles_match_oracle(gpu, m, n, k, gs):
     """mtp_qmm_affine4_tiles at the edges of its row tiles (64), column groups
