@@ -1374,7 +1374,16 @@ __global__ __launch_bounds__(kSampThreads) void wide_hist(const float* __restric
     __syncthreads();
     if (tid == 0) {
       const int n = n_chunks - c0 < kSampThreads ? n_chunks - c0 : kSampThreads;
-      for (int i = 0; i < n; ++i) S = fma(s_sum[i], s_exp[i], S);
+      for (int i = 0; i < n; i += 8) {   // (zeros past n: they leave S as it is)
+        double a[8], e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          a[j] = s_sum[i + j];
+          e[j] = s_exp[i + j];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) S = fma(a[j], e[j], S);
+      }
     }
     __syncthreads();
   }
