@@ -78,9 +78,10 @@ int mtp_chunk_sums(const void* x, int M, int K, float* out, void* stream);
 /* The cross-row lane's matmul with its precomputed chunk sums
  * (mtplx/verify_crossrow.py:249 crossrow_qmm(..., xsums=make_chunk_sums(x))):
  * 4-bit affine, group 32 or 64, 1 <= M <= 8, K a multiple of 512; x bf16
- * [M, K], xsums the mtp_chunk_sums table of x; y bf16 [M, N]. Each 32-k
- * block's bias term b * sum(x) reads its sum from the table (two 16-value
- * slices) instead of re-summing the staged x; otherwise as mtp_qmv_affine. */
+ * [M, K], xsums the mtp_chunk_sums table of x; y bf16 [M, N]. Each
+ * group's bias term b * sum(x) takes its sum from the table (its 16-value
+ * slices); otherwise as mtp_qmv_affine, which also forms the group sums that
+ * take 128 s off the fields' 128 + q (as it does without a table). */
 int mtp_crossrow_qmm(const void* x, const float* xsums, const void* w, const void* scales, const void* biases,
                      void* y, int M, int N, int K, int group_size, void* stream);
 

@@ -4,7 +4,8 @@
 //
 // What bounds it: the matrix cores, once every weight is used by enough rows;
 // in 64-row launches of qmm_rows_kernel each launch reads all weights again
-// on at most 136 of the 256 CUs. Here one launch covers all row tiles:
+// with a workgroup per 128 columns (136 for 17408) on 256 CUs. Here one launch
+// covers all row tiles:
 //  * a workgroup of 4 waves computes 64 rows x 128 columns, a wave 64 x 32 on
 //    v_mfma_f32_32x32x16_bf16: per 64-k group 8 MFMAs (256 cycles) against 28
 //    VALU instructions that unpack the weights and 32 that scale the group's
@@ -22,8 +23,8 @@
 //    runs on XCD b % 8), so the row tiles share its L2's weights;
 //  * small grids are split by K (tiles_split), the parts' fp32 sums added in part
 //    order by a second kernel.
-// Measured: 512 rows, 17408 x 5120: 129.7 us (704 TFLOP/s; 274.7 in 64-row
-// launches), 2048 rows: 465 us (785; 1080).
+// Measured: 512 rows, 17408 x 5120: 118-122 us (750-770 TFLOP/s; 272 in 64-row
+// launches), 2048 rows: 453 us (806; 1080 then).
 #include "qmv_args.hpp"
 
 namespace mtp {
@@ -112,8 +113,8 @@ __global__ __launch_bounds__(kTiThreads, 2) void qmm_tiles_kernel(TilesParams p)
     r.sb = *reinterpret_cast<const uint4*>(sl + off);
   };
   // x of quad q: wave instruction t holds rows 2 t, 2 t + 1 (16-byte piece kc of
-  // row m at slot kc ^ (m & 15)); wave w takes t = w, w + 4, .., and its 16 rows'
-  // sums with one more (half the lanes; the others repeat them).
+  // row m at slot kc ^ (m & 15)); wave w takes t = w, w + 4, .., and waves 0 and 1
+  // the sums of 32 rows each with one more.
   const uint16_t* xp[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {

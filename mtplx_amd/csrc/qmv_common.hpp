@@ -361,8 +361,8 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Direct-to-LDS loads issued as assembly: lane i's 16 (or 4) bytes go to lds +
-// 16 i (4 i); lds is a wave-uniform LDS byte address (lds_addr). With the
+// Direct-to-LDS loads issued as assembly: lane i's 16 bytes go to lds + 16 i;
+// lds is a wave-uniform LDS byte address (lds_addr). With the
 // builtin the compiler takes every later LDS read of the kernel for one that
 // may need the data and waits for all loads in flight (vmcnt(0)) at the first
 // LDS read after it, which drains a double buffer at every step. These have
@@ -381,10 +381,6 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t l
 }
 __device__ __forceinline__ void dma16(const void* lane_ptr, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(lds), "v"(lane_ptr) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const void* lane_ptr, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
                :: "s"(lds), "v"(lane_ptr) : "memory", "m0");
 }
 #pragma clang diagnostic pop

@@ -44,9 +44,9 @@
 // Measured (MI355X, weights from HBM): 8-bit group 64, 17408 x 5120, 4 rows:
 // 24 us (3.9 TB/s; 138 us with one lane per column on the VALU), 65536 x 5120:
 // 66 us (5.4 TB/s). 256 experts of 2 x 1536 x 4096, 16 rows x 8 (59 of them
-// with 1..4 rows): gate|up 90 us and down 48 us (4.4 and 4.2 TB/s) for those;
-// all experts 355 and 240 us before, each lane reading 16 bytes of its own
-// row. A wave's own instructions bound it there: with one wave per SIMD, two,
+// with 1..4 rows): gate|up 90 us and down 48 us (4.4 and 4.2 TB/s) for those, 99
+// and 55 with the others; 355 and 240 us before, each lane reading 16 bytes of
+// its own row. A wave's own instructions bound it there: with one wave per SIMD, two,
 // three or four stages all take 131 us (gate|up), with two waves 92.
 #pragma once
 
@@ -145,7 +145,8 @@ __device__ __forceinline__ void group_vals(const unsigned char* at, float (&o)[G
 // an expert has more rows than m_hi.
 // VEC: scales straight to LDS, and x 16-byte aligned (else scales element by
 // element, and x too where it is not aligned). XS: the bias term
-// takes its group sums from the caller's chunk-sum table (p.xsums).
+// takes its group sums from the caller's chunk-sum table (p.xsums); those that
+// take 128 s off the fields' 128 + q are the MFMA's as in the others.
 template <int BITS, int GS, int R, bool DUAL, bool VEC, bool XS, int NW, int KS, int ND>
 __device__ __forceinline__ bool inplace_body(const InplaceParams& p, unsigned char* const lds_base, int bid, int m_lo,
                                              int m_hi) {

@@ -1263,8 +1263,8 @@ __global__ __launch_bounds__(kWideThreads) void wide_law_kernel(const float* __r
 // The same law over many workgroups, for rows of more than two chunks. One
 // workgroup per row leaves most of the chip idle (28 rows on 256 CUs) and walks
 // a row in 149 rounds of block scans: 557 us for 28 rows of 151936. Here, with
-// the same ids and probabilities bit for bit, 26 + 15 + 10 + 12 us (the accept
-// step of four requests of depth 3: 597-612 -> 121-138 us):
+// the same ids and probabilities bit for bit, 25 + 15 + 10 + 11 us (the accept
+// step of four requests of depth 3: 597-612 -> 111-138 us):
 //  1. wide_hist: per chunk, the count and fixed-point mass of each bin of the
 //     distance from the row's maximum (bins are monotone in the logit; integer
 //     sums, so the order of the additions does not matter);

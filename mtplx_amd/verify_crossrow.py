@@ -6,10 +6,12 @@
 ``make_chunk_sums`` fills the reference's table layout on the GPU
 (``mtp_chunk_sums``: per 512-k block and lane, the 16-value slice sum of
 each row, stride 8). ``crossrow_qmm`` with a table runs ``mtp_crossrow_qmm``,
-whose 32-k block finishes read their activation sums from the table (two
-slices per block) instead of re-summing the staged x; without one it runs
-the verify matmul, which forms the sums while staging x. Both meet the same
-oracle bar; the two sum orders differ only in fp32 rounding.
+whose bias terms take their activation sums from the table (a group's
+slices); without one it runs the verify matmul, which forms the sums itself.
+Both meet the same oracle bar; the two sum orders differ only in fp32
+rounding. The table is the reference's interface, not a saving here: fields
+enter the matrix cores as 128 + q, so the in-place matmul sums every group of
+x beside its products in any case.
 """
 
 from __future__ import annotations
